@@ -133,56 +133,100 @@ __global__ __launch_bounds__(256) void group_len_kernel(const uint32_t *__restri
   if (g < ngroups) aw[g] = slen[g * 64];
 }
 
-// One wave per (sub-)group w: lane l holds chunk l % tpr of sorted row
+// One block per (sub-)group w: lane l holds chunk l % tpr of sorted row
 // row_off[w] + l / tpr (WPK1: tpr 1, rows 64 w + l); its slots are
 // warp_offsets[w] + l + 64 i, i < A_w; slots past the chunk are pads (0, col 0).
+// The rows' entries are read kFillSteps at a time, 256 bytes of values per row
+// together, turned around in LDS and written a step (64 slots) at a time, so
+// reads, padded arrays and the CSR-to-slot map are all whole lines.  (A lane
+// per row walking its own entries read 64 scattered lines per load and wrote
+// the map 4 bytes to a line: hex elasticity 40^3, 16M entries, 725 us against
+// 107.)
+constexpr int kFillSteps = 32;
+constexpr int kFillThreads = 256;
+
 template <class T>
-__global__ __launch_bounds__(256) void fill_kernel(
+__global__ __launch_bounds__(kFillThreads) void fill_kernel(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ colind,
     const double *__restrict__ vals, const int32_t *__restrict__ row_map,
     const int32_t *__restrict__ row_map_inv, const int64_t *__restrict__ wo,
     const uint32_t *__restrict__ aw, const uint32_t *__restrict__ tpr_a,
-    const uint32_t *__restrict__ row_off, int32_t ngroups, int32_t nznrows, T *__restrict__ pv,
+    const uint32_t *__restrict__ row_off, int32_t nznrows, T *__restrict__ pv,
     int32_t *__restrict__ pc, int32_t *__restrict__ pkr, uint32_t *__restrict__ slot_of_nz) {
-  const int32_t lane = threadIdx.x & 63;
-  const int32_t w = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (w >= ngroups) return;
+  constexpr int PER = kFillSteps * 64 / kFillThreads;
+  __shared__ int32_t first[64], count[64];        // each lane's first CSR entry, entries
+  __shared__ T sv[64][kFillSteps + 1];            // odd row length: the turned reads spread
+  __shared__ int32_t sc[64][kFillSteps + 1];
+  const int32_t w = blockIdx.x;
+  const int32_t tid = threadIdx.x;
   const uint32_t A = aw[w];
-  const uint32_t tpr = tpr_a ? tpr_a[w] : 1u;
-  const uint32_t p = (tpr_a ? row_off[w] : (uint32_t)w * 64u) + (uint32_t)lane / tpr;
-  const uint32_t chunk = (uint32_t)lane & (tpr - 1);
-  int32_t rb = 0, n = 0;
-  if (p < (uint32_t)nznrows) {
-    const int32_t r = row_map[p];
-    const int32_t b1 = rowptr[r + 1];
-    rb = rowptr[r] + (int32_t)(chunk * A);
-    n = max(0, min(b1 - rb, (int32_t)A));
-  }
-  const int64_t base = wo[w] + lane;
-  for (uint32_t i = 0; i < A; i++) {
-    const int64_t slot = base + (int64_t)i * 64;
-    if ((int32_t)i < n) {
-      const int32_t e = rb + (int32_t)i;
-      const int32_t c = colind[e];
-      pv[slot] = (T)vals[e];
-      pc[slot] = c;
-      if (pkr) pkr[slot] = row_map_inv[c];
-      slot_of_nz[e] = (uint32_t)slot;
-    } else {
-      pv[slot] = T(0);
-      pc[slot] = 0;
-      if (pkr) pkr[slot] = 0;
+  if (tid < 64) {
+    const uint32_t tpr = tpr_a ? tpr_a[w] : 1u;
+    const uint32_t p = (tpr_a ? row_off[w] : (uint32_t)w * 64u) + (uint32_t)tid / tpr;
+    const uint32_t chunk = (uint32_t)tid & (tpr - 1);
+    int32_t rb = 0, n = 0;
+    if (p < (uint32_t)nznrows) {
+      const int32_t r = row_map[p];
+      const int32_t b1 = rowptr[r + 1];
+      rb = rowptr[r] + (int32_t)(chunk * A);
+      n = max(0, min(b1 - rb, (int32_t)A));
     }
+    first[tid] = rb;
+    count[tid] = n;
+  }
+  __syncthreads();
+  const int64_t base = wo[w];
+  for (uint32_t i0 = 0; i0 < A; i0 += kFillSteps) {
+    T v[PER];
+    int32_t c[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+      const int32_t l = (tid + j * kFillThreads) / kFillSteps;
+      const int32_t i = (int32_t)i0 + tid % kFillSteps;
+      v[j] = T(0);
+      c[j] = 0;
+      if (i < count[l]) {
+        const int32_t e = first[l] + i;
+        v[j] = (T)vals[e];
+        c[j] = colind[e];
+        slot_of_nz[e] = (uint32_t)(base + l + 64 * (int64_t)i);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+      const int32_t l = (tid + j * kFillThreads) / kFillSteps;
+      sv[l][tid % kFillSteps] = v[j];
+      sc[l][tid % kFillSteps] = c[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+      const int32_t l = tid & 63, t = (tid + j * kFillThreads) >> 6;
+      const uint32_t i = i0 + (uint32_t)t;
+      if (i < A) {
+        const int64_t slot = base + l + 64 * (int64_t)i;
+        const int32_t col = sc[l][t];
+        pv[slot] = sv[l][t];
+        pc[slot] = col;
+        if (pkr) pkr[slot] = (int32_t)i < count[l] ? row_map_inv[col] : 0;
+      }
+    }
+    __syncthreads();
   }
 }
 
 // ---------------------------------------------------------------- x windows
-// The windows of build_windows (scan.cpp), built on the device: one block per
-// group sorts the group's slot keys (the entry's column, -1 for a pad) in LDS,
-// counts the distinct ones (pass 1), then writes them and each slot's
-// position among them (pass 2).  Groups of more than kWinSlots slots are not
-// handled here: the engine then has no windows.
+// The windows of build_windows (scan.cpp), built on the device, one block per
+// group: the distinct slot keys (the entry's column, -1 for a pad) are counted
+// (pass 1), then written with each slot's position among them (pass 2).  Where
+// the group's columns span at most kWinBits (every banded ordering) the keys
+// set bits of an LDS bitmap, and a key's position is the number of bits below
+// its own: the words' running counts plus one popcount.  Wider groups sort
+// their keys in LDS.  (Sorting every group took 1.01 + 1.38 ms on hex elasticity
+// 40^3, 3,231 groups of 5,184 slots; the bitmap BIT_US.)  Groups of more than
+// kWinSlots slots are not handled here: the engine then has no windows.
 constexpr int32_t kWinSlots = 8192;
+constexpr int32_t kWinBits = kWinSlots * 32;  // the bitmap takes the sort's LDS
 constexpr int kWinThreads = 256;
 
 struct WinBuild {
@@ -192,17 +236,11 @@ struct WinBuild {
   int32_t nznrows;
 };
 
-// Sorted keys of group g in keys[0, N) (INT_MAX past the S slots); returns S,
-// or -1 when the group has too many slots.
-__device__ int32_t sort_group_keys(const WinBuild &b, int32_t g, int32_t *keys, int32_t *lane_n,
-                                   int32_t &N) {
-  const uint32_t A = b.aw[g];
-  const int64_t S64 = (int64_t)A * 64;
-  if (S64 > kWinSlots) return -1;
-  const int32_t S = (int32_t)S64;
+// Entries of each lane of group g (the fill kernel's chunk rule).
+__device__ void lane_entries(const WinBuild &b, int32_t g, int32_t *lane_n) {
   const int32_t tid = threadIdx.x;
   if (tid < 64) {
-    // entries of lane tid (the fill kernel's chunk rule)
+    const uint32_t A = b.aw[g];
     const uint32_t tpr = b.tpr ? b.tpr[g] : 1u;
     const uint32_t p = (b.tpr ? b.row_off[g] : (uint32_t)g * 64u) + (uint32_t)tid / tpr;
     const uint32_t chunk = (uint32_t)tid & (tpr - 1);
@@ -214,9 +252,15 @@ __device__ int32_t sort_group_keys(const WinBuild &b, int32_t g, int32_t *keys, 
     }
     lane_n[tid] = n;
   }
+  __syncthreads();
+}
+
+// Sorted keys of group g in keys[0, N) (INT_MAX past the S slots).
+__device__ void sort_group_keys(const WinBuild &b, int32_t g, int32_t S, int32_t *keys,
+                                const int32_t *lane_n, int32_t &N) {
+  const int32_t tid = threadIdx.x;
   N = 64;
   while (N < S) N <<= 1;
-  __syncthreads();
   const int64_t base = b.wo[g];
   for (int32_t t = tid; t < N; t += kWinThreads)
     keys[t] = t < S ? ((t >> 6) < lane_n[t & 63] ? b.cols[base + t] : -1) : INT32_MAX;
@@ -235,51 +279,61 @@ __device__ int32_t sort_group_keys(const WinBuild &b, int32_t g, int32_t *keys, 
       }
       __syncthreads();
     }
-  return S;
 }
 
-__global__ __launch_bounds__(kWinThreads) void window_count_kernel(WinBuild b, int32_t *count) {
-  __shared__ int32_t keys[kWinSlots];
-  __shared__ int32_t lane_n[64];
-  __shared__ int32_t part[kWinThreads];
-  const int32_t g = blockIdx.x;
-  int32_t N = 0;
-  const int32_t S = sort_group_keys(b, g, keys, lane_n, N);
-  if (S < 0) {
-    if (threadIdx.x == 0) count[g] = -1;
-    return;
-  }
-  int32_t c = 0;
-  for (int32_t t = threadIdx.x; t < N; t += kWinThreads)
-    c += keys[t] != INT32_MAX && (t == 0 || keys[t] != keys[t - 1]);
-  part[threadIdx.x] = c;
-  __syncthreads();
-  for (int o = kWinThreads / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) part[threadIdx.x] += part[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) count[g] = part[0] > kMaxWindow ? -1 : part[0];
-}
-
-__global__ __launch_bounds__(kWinThreads) void window_write_kernel(WinBuild b, const uint32_t *off,
-                                                                   int32_t *win_cols,
-                                                                   int32_t *win_cols_kr,
-                                                                   uint16_t *win_idx) {
-  __shared__ int32_t keys[kWinSlots];
-  __shared__ int32_t uniq[kMaxWindow];
-  __shared__ int32_t lane_n[64];
-  __shared__ int32_t part[kWinThreads];
-  const int32_t g = blockIdx.x;
+// The least and greatest column of the group's entries and whether it has a
+// pad, over the whole block (red: kWinThreads ints).
+struct Span {
+  int32_t lo, hi, pad;
+};
+__device__ Span group_span(const WinBuild &b, int64_t base, int32_t S, const int32_t *lane_n, int32_t *red) {
   const int32_t tid = threadIdx.x;
-  int32_t N = 0;
-  const int32_t S = sort_group_keys(b, g, keys, lane_n, N);
-  if (S < 0) return;  // not reached: the host builds windows only when every group fits
-  // ranks of the distinct keys: each thread counts a contiguous chunk of the
-  // sorted keys, then an inclusive scan of the chunk counts
-  const int32_t per = N / kWinThreads > 0 ? N / kWinThreads : 1;
-  const int32_t t0 = min(N, tid * per), t1 = min(N, t0 + per);
-  int32_t c = 0;
-  for (int32_t t = t0; t < t1; t++) c += keys[t] != INT32_MAX && (t == 0 || keys[t] != keys[t - 1]);
+  int32_t lo = INT32_MAX, hi = -1, pad = 0;
+  for (int32_t t = tid; t < S; t += kWinThreads) {
+    if ((t >> 6) < lane_n[t & 63]) {
+      const int32_t c = b.cols[base + t];
+      lo = min(lo, c);
+      hi = max(hi, c);
+    } else {
+      pad = 1;
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, __shfl_xor(lo, o));
+    hi = max(hi, __shfl_xor(hi, o));
+    pad |= __shfl_xor(pad, o);
+  }
+  if ((tid & 63) == 0) {
+    red[tid >> 6] = lo;
+    red[8 + (tid >> 6)] = hi;
+    red[16 + (tid >> 6)] = pad;
+  }
+  __syncthreads();
+  for (int w = 0; w < kWinThreads / 64; w++) {
+    lo = min(lo, red[w]);
+    hi = max(hi, red[8 + w]);
+    pad |= red[16 + w];
+  }
+  __syncthreads();
+  return {lo, hi, pad};
+}
+
+// Sets the bit of every entry's column in bits[0, words) (bit 0: column lo).
+__device__ void group_bits(const WinBuild &b, int64_t base, int32_t S, const int32_t *lane_n, int32_t lo,
+                           int32_t words, uint32_t *bits) {
+  for (int32_t t = threadIdx.x; t < words; t += kWinThreads) bits[t] = 0;
+  __syncthreads();
+  for (int32_t t = threadIdx.x; t < S; t += kWinThreads)
+    if ((t >> 6) < lane_n[t & 63]) {
+      const uint32_t k = (uint32_t)(b.cols[base + t] - lo);
+      atomicOr(&bits[k >> 5], 1u << (k & 31));
+    }
+  __syncthreads();
+}
+
+// Inclusive sum of every thread's c over the block (part: kWinThreads ints).
+__device__ int32_t block_scan(int32_t c, int32_t *part) {
+  const int32_t tid = threadIdx.x;
   part[tid] = c;
   __syncthreads();
   for (int o = 1; o < kWinThreads; o <<= 1) {
@@ -288,33 +342,135 @@ __global__ __launch_bounds__(kWinThreads) void window_write_kernel(WinBuild b, c
     part[tid] += v;
     __syncthreads();
   }
-  int32_t rank = part[tid] - c;
-  const uint32_t w0 = off[g];
-  for (int32_t t = t0; t < t1; t++) {
-    const int32_t k = keys[t];
-    if (k != INT32_MAX && (t == 0 || k != keys[t - 1])) {
-      uniq[rank] = k;
-      win_cols[w0 + rank] = k < 0 ? 0 : k;
-      if (win_cols_kr) win_cols_kr[w0 + rank] = k < 0 ? 0 : b.row_map_inv[k];
-      rank++;
+  return part[tid];
+}
+
+// count[g]: distinct keys, or -1; words[g]: bitmap words of the group, or
+// INT32_MAX where its keys have to be sorted.
+__global__ __launch_bounds__(kWinThreads) void window_count_kernel(WinBuild b, int32_t *count, int32_t *nwords) {
+  __shared__ int32_t keys[kWinSlots];
+  __shared__ int32_t lane_n[64];
+  __shared__ int32_t part[kWinThreads];
+  const int32_t g = blockIdx.x;
+  const int64_t S64 = (int64_t)b.aw[g] * 64;
+  if (S64 > kWinSlots) {
+    if (threadIdx.x == 0) {
+      count[g] = -1;
+      nwords[g] = 0;
     }
+    return;
   }
-  __syncthreads();
-  // each slot's position among the distinct keys (ascending; a pad's key -1,
-  // when present, is the first)
-  const int32_t n = part[kWinThreads - 1];
+  const int32_t S = (int32_t)S64;
   const int64_t base = b.wo[g];
-  for (int32_t t = tid; t < S; t += kWinThreads) {
-    const int32_t key = (t >> 6) < lane_n[t & 63] ? b.cols[base + t] : -1;
-    int32_t lo = 0, hi = n;
-    while (lo < hi) {
-      const int32_t mid = (lo + hi) >> 1;
-      if (uniq[mid] < key)
-        lo = mid + 1;
-      else
-        hi = mid;
+  lane_entries(b, g, lane_n);
+  const Span sp = group_span(b, base, S, lane_n, part);
+  int32_t c = 0;
+  if (sp.hi - sp.lo < kWinBits) {
+    const int32_t words = (sp.hi - sp.lo + 32) >> 5;
+    uint32_t *bits = reinterpret_cast<uint32_t *>(keys);
+    group_bits(b, base, S, lane_n, sp.lo, words, bits);
+    for (int32_t t = threadIdx.x; t < words; t += kWinThreads) c += __popc(bits[t]);
+    if (threadIdx.x == 0) c += sp.pad;
+  } else {
+    int32_t N = 0;  // the keys in LDS: S rounded up to a power of two
+    sort_group_keys(b, g, S, keys, lane_n, N);
+    for (int32_t t = threadIdx.x; t < N; t += kWinThreads)
+      c += keys[t] != INT32_MAX && (t == 0 || keys[t] != keys[t - 1]);
+  }
+  const int32_t total = block_scan(c, part);
+  if (threadIdx.x == kWinThreads - 1) {
+    count[g] = total > kMaxWindow ? -1 : total;
+    nwords[g] = sp.hi - sp.lo < kWinBits ? (sp.hi - sp.lo + 32) >> 5 : INT32_MAX;
+  }
+}
+
+// WIDE: some group's keys have to be sorted (dynamic LDS for kWinSlots keys);
+// otherwise 6 bytes of dynamic LDS for each of nw bitmap words.
+template <bool WIDE>
+__global__ __launch_bounds__(kWinThreads) void window_write_kernel(WinBuild b, const uint32_t *off,
+                                                                   int32_t *win_cols,
+                                                                   int32_t *win_cols_kr,
+                                                                   uint16_t *win_idx, int32_t nw) {
+  extern __shared__ int32_t keys[];
+  uint16_t *below = reinterpret_cast<uint16_t *>(keys + nw);  // bits in the words before
+  __shared__ int32_t uniq[WIDE ? kMaxWindow : 1];
+  __shared__ int32_t lane_n[64];
+  __shared__ int32_t part[kWinThreads];
+  const int32_t g = blockIdx.x;
+  const int32_t tid = threadIdx.x;
+  const int32_t S = (int32_t)b.aw[g] * 64;  // at most kWinSlots: the host builds windows only then
+  const int64_t base = b.wo[g];
+  const uint32_t w0 = off[g];
+  lane_entries(b, g, lane_n);
+  const Span sp = group_span(b, base, S, lane_n, part);
+  if (!WIDE || sp.hi - sp.lo < kWinBits) {
+    const int32_t words = (sp.hi - sp.lo + 32) >> 5;
+    uint32_t *bits = reinterpret_cast<uint32_t *>(keys);
+    group_bits(b, base, S, lane_n, sp.lo, words, bits);
+    const int32_t per = (words + kWinThreads - 1) / kWinThreads;
+    const int32_t t0 = min(words, tid * per), t1 = min(words, t0 + per);
+    int32_t c = 0;
+    for (int32_t t = t0; t < t1; t++) c += __popc(bits[t]);
+    int32_t rank = block_scan(c, part) - c + sp.pad;  // a pad's key is the first
+    if (tid == 0 && sp.pad) {
+      win_cols[w0] = 0;
+      if (win_cols_kr) win_cols_kr[w0] = 0;
     }
-    win_idx[base + t] = (uint16_t)lo;
+    for (int32_t t = t0; t < t1; t++) {
+      below[t] = (uint16_t)rank;
+      for (uint32_t m = bits[t]; m; m &= m - 1) {
+        const int32_t k = sp.lo + 32 * t + (__ffs((int)m) - 1);
+        win_cols[w0 + rank] = k;
+        if (win_cols_kr) win_cols_kr[w0 + rank] = b.row_map_inv[k];
+        rank++;
+      }
+    }
+    __syncthreads();
+    for (int32_t t = tid; t < S; t += kWinThreads) {
+      int32_t p = 0;
+      if ((t >> 6) < lane_n[t & 63]) {
+        const uint32_t k = (uint32_t)(b.cols[base + t] - sp.lo);
+        p = below[k >> 5] + __popc(bits[k >> 5] & ((1u << (k & 31)) - 1u));
+      }
+      win_idx[base + t] = (uint16_t)p;
+    }
+    return;
+  }
+  if constexpr (WIDE) {
+    int32_t N = 0;
+    sort_group_keys(b, g, S, keys, lane_n, N);
+    // ranks of the distinct keys: each thread counts a contiguous chunk of the
+    // sorted keys, then an inclusive scan of the chunk counts
+    const int32_t per = N / kWinThreads > 0 ? N / kWinThreads : 1;
+    const int32_t t0 = min(N, tid * per), t1 = min(N, t0 + per);
+    int32_t c = 0;
+    for (int32_t t = t0; t < t1; t++) c += keys[t] != INT32_MAX && (t == 0 || keys[t] != keys[t - 1]);
+    int32_t rank = block_scan(c, part) - c;
+    for (int32_t t = t0; t < t1; t++) {
+      const int32_t k = keys[t];
+      if (k != INT32_MAX && (t == 0 || k != keys[t - 1])) {
+        uniq[rank] = k;
+        win_cols[w0 + rank] = k < 0 ? 0 : k;
+        if (win_cols_kr) win_cols_kr[w0 + rank] = k < 0 ? 0 : b.row_map_inv[k];
+        rank++;
+      }
+    }
+    __syncthreads();
+    // each slot's position among the distinct keys (ascending; a pad's key -1,
+    // when present, is the first)
+    const int32_t n = part[kWinThreads - 1];
+    for (int32_t t = tid; t < S; t += kWinThreads) {
+      const int32_t key = (t >> 6) < lane_n[t & 63] ? b.cols[base + t] : -1;
+      int32_t lo = 0, hi = n;
+      while (lo < hi) {
+        const int32_t mid = (lo + hi) >> 1;
+        if (uniq[mid] < key)
+          lo = mid + 1;
+        else
+          hi = mid;
+      }
+      win_idx[base + t] = (uint16_t)lo;
+    }
   }
 }
 
@@ -333,10 +489,9 @@ template <class T>
 void launch_fill(const DevLayout &D, const int32_t *rowptr, const int32_t *colind,
                  const double *vals, hipStream_t s) {
   if (!D.ngroups) return;
-  hipLaunchKernelGGL(fill_kernel<T>, dim3((uint32_t)((D.ngroups + 3) / 4)), dim3(256), 0, s,
-                     rowptr, colind, vals, D.row_map, D.row_map_inv, D.warp_offsets,
-                     D.max_nz_rows, D.tpr, D.row_off, D.ngroups, D.nznrows,
-                     static_cast<T *>(D.vals), D.cols, D.cols_kr, D.slot_of_nz);
+  hipLaunchKernelGGL(fill_kernel<T>, dim3((uint32_t)D.ngroups), dim3(kFillThreads), 0, s, rowptr,
+                     colind, vals, D.row_map, D.row_map_inv, D.warp_offsets, D.max_nz_rows, D.tpr,
+                     D.row_off, D.nznrows, static_cast<T *>(D.vals), D.cols, D.cols_kr, D.slot_of_nz);
   hip_check(hipGetLastError(), "fill");
 }
 
@@ -458,15 +613,17 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
   if (G) {
     WinBuild wb{rowptr, D.row_map, D.row_map_inv, D.cols, D.warp_offsets, D.max_nz_rows,
                 D.tpr, D.row_off, nznrows};
-    int32_t *dcount = dev_alloc<int32_t>(E, G);
-    hipLaunchKernelGGL(window_count_kernel, dim3((uint32_t)G), dim3(kWinThreads), 0, s, wb, dcount);
+    int32_t *dcount = dev_alloc<int32_t>(E, 2 * (int64_t)G);
+    hipLaunchKernelGGL(window_count_kernel, dim3((uint32_t)G), dim3(kWinThreads), 0, s, wb, dcount,
+                       dcount + G);
     hip_check(hipGetLastError(), "window count");
-    const std::vector<int32_t> cnt = download(dcount, G, s);
+    const std::vector<int32_t> cnt = download(dcount, 2 * (int64_t)G, s);
     bool fits = true;
     std::vector<uint32_t> off((size_t)G + 1, 0);
-    int32_t most = 0;
+    int32_t most = 0, words = 0;
     for (int32_t g = 0; g < G && fits; g++) {
       if (cnt[g] < 0) fits = false;
+      words = std::max(words, cnt[(size_t)G + g]);
       off[g + 1] = off[g] + (uint32_t)std::max(cnt[g], 0);
       most = std::max(most, cnt[g]);
     }
@@ -475,8 +632,12 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
       D.win_cols = dev_alloc<int32_t>(E, off[G]);
       D.win_cols_kr = kr ? dev_alloc<int32_t>(E, off[G]) : nullptr;
       D.win_idx = dev_alloc<uint16_t>(E, D.allocate_nz);
-      hipLaunchKernelGGL(window_write_kernel, dim3((uint32_t)G), dim3(kWinThreads), 0, s, wb,
-                         D.win_off, D.win_cols, D.win_cols_kr, D.win_idx);
+      if (words > kWinSlots)  // the words of the groups that have a bitmap, or the sort's keys
+        hipLaunchKernelGGL(window_write_kernel<true>, dim3((uint32_t)G), dim3(kWinThreads), 6 * kWinSlots, s,
+                           wb, D.win_off, D.win_cols, D.win_cols_kr, D.win_idx, kWinSlots);
+      else
+        hipLaunchKernelGGL(window_write_kernel<false>, dim3((uint32_t)G), dim3(kWinThreads),
+                           6 * (size_t)words, s, wb, D.win_off, D.win_cols, D.win_cols_kr, D.win_idx, words);
       hip_check(hipGetLastError(), "window write");
       hip_check(hipStreamSynchronize(s), "window write");
       D.win_max = most;
