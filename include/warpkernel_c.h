@@ -346,7 +346,11 @@ typedef struct wk_launch {
                               right-hand sides through a window of that
                               many values per column; the rest of k (fewer
                               than one tile), and engines it does not fit,
-                              run as 4; 7 (k_tile 1, engines with node
+                              run as 4; where neighbouring rows share their
+                              columns (block matrices, WPK1, at most 84
+                              steps) FP64 engines, and FP32 ones with
+                              WK_ACC_F64, run all of k on the matrix cores
+                              instead, each row's sum in the same order; 7 (k_tile 1, engines with node
                               windows; run, run_x and the residual): as 5, with a
                               window of node entries (three x values at
                               columns 3n .. 3n+2, or one column thrice for
@@ -432,7 +436,9 @@ int wk_tune(wk_engine *engine, int32_t op, const wk_launch *base, const void *x_
             wk_launch *best, float *best_ms);
 
 /* Read / replace the configuration the engine uses for (op, k) when cfg is
- * NULL (before tuning: a choice from the layout's mean row length). */
+ * NULL (before tuning: a choice from the layout; FP32 engines get WK_ACC_F64
+ * where the matrix cores sum, which is closer to the exact result than
+ * WK_ACC_TWOSUM). */
 int wk_engine_get_launch(const wk_engine *engine, int32_t op, int32_t k, wk_launch *cfg);
 int wk_engine_set_launch(wk_engine *engine, int32_t op, int32_t k, const wk_launch *cfg);
 

@@ -47,6 +47,7 @@ void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double 
   D.variant = L.variant;
   D.W = L.W;
   D.nrows = L.nrows;
+  D.ncols = L.ncols;
   D.nznrows = L.nznrows;
   D.ngroups = L.nwarps;
   D.allocate_nz = L.allocate_nz;
@@ -103,6 +104,7 @@ void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double 
         hip_check(hipStreamSynchronize(s), "upload");
       }
       build_packed_positions(E, D, s);
+      build_row_sets(E, D, s);
     } else {
       D.win_max = 0;
     }

@@ -505,6 +505,7 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
   D.variant = variant;
   D.W = 64;
   D.nrows = nrows;
+  D.ncols = ncols;
 
   // 1. check the CSR, find the longest row
   const int64_t work = std::max<int64_t>(nrows, nnz);
@@ -643,6 +644,7 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
       D.win_max = most;
       D.win_total = off[G];
       build_packed_positions(E, D, s);
+      build_row_sets(E, D, s);
     }
   }
 

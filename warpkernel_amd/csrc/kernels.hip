@@ -33,17 +33,6 @@ namespace {
 
 constexpr int kMaxThreads = 512;
 
-// ----------------------------------------------------------- block mapping
-// Workgroups are handed to the 8 XCDs round-robin by id.  With remap, the
-// blocks an XCD receives cover one contiguous range of work ids, so the x
-// window of neighbouring groups stays in that XCD's L2.
-__device__ __forceinline__ int32_t work_id(int32_t b, int32_t nwork, int32_t remap) {
-  if (!remap) return b;
-  const int32_t q = nwork >> 3, r = nwork & 7;
-  const int32_t xcd = b & 7, idx = b >> 3;
-  return xcd * q + (xcd < r ? xcd : r) + idx;
-}
-
 // ----------------------------------------------------------------- kernel
 // One group's slice of a wave: base offset, steps, lanes per row, first row.
 struct GroupMeta {
@@ -1245,6 +1234,14 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
   }
 
   int32_t j0 = 0;
+  // stage 6 on layouts with row sets (FP64, or FP32 values with FP64 sums): the
+  // matrix cores, all of k in one launch
+  if (cfg.stage_lds == 6 && rpl == 1 && cfg.nontemporal) {
+    a.x = x;
+    a.y = y;
+    a.b = b;
+    if (launch_rowsets(D, prec, out, a, k, cfg.xcd_remap ? 1 : 0, stream)) return;
+  }
   // stage 6: the group's values in registers, one pass per 32-byte k-tile
   // (4 FP64 or 8 FP32 right-hand sides), all passes of a group in one wave;
   // the rest of k (fewer than one tile) continues below

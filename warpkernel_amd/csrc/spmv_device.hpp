@@ -25,6 +25,17 @@ __device__ __forceinline__ T ld_stream(const T *p) {
     return *p;
 }
 
+// ----------------------------------------------------------- block mapping
+// Workgroups are handed to the 8 XCDs round-robin by id.  With remap, the
+// blocks an XCD receives cover one contiguous range of work ids, so the x
+// window of neighbouring groups stays in that XCD's L2.
+__device__ __forceinline__ int32_t work_id(int32_t b, int32_t nwork, int32_t remap) {
+  if (!remap) return b;
+  const int32_t q = nwork >> 3, r = nwork & 7;
+  const int32_t xcd = b & 7, idx = b >> 3;
+  return xcd * q + (xcd < r ? xcd : r) + idx;
+}
+
 // ---------------------------------------------------------------- precision
 struct PF64 {
   using V = double;

@@ -351,6 +351,25 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k) {
       }
     }
   }
+  if (D.rs_waves > 0 && win_ok && k >= 5 && (dtype == WK_F64 || k >= 9 || D.ngroups < 8192)) {
+    // row sets on the matrix cores (stage 6, rowsets.hip), all of k in one
+    // launch.  Hex elasticity, FP64: 32^3 k=5 18.1 us against 36.4, k=8 18.7
+    // against 30.9, k=16 25.1 against 58.4, k=32 38.4 against 100; 64^3 k=5
+    // 176 against 194, k=8 181 against 204, k=16 248 against 421, k=32 382
+    // against 803.  Up to k = 4 the windows read less: 32^3 k=4 17.5 either
+    // way, 64^3 175 against 118.  FP32 values: FP64 sums, exact products, so
+    // the result is closer to the exact one than the compensated FP32 sums'
+    // (1e-16 against 2e-14 normwise on 32^3) at 13.7 us against 23.5 (32^3
+    // k=8; 36.4 against 69 on 48^3); the 64^3 layout (12,874 groups) keeps
+    // its windows up to k = 8.
+    c.stage_lds = 6;
+    c.unroll = 8;
+    c.k_tile = 8;
+    c.waves_per_block = 1;
+    c.rows_per_lane = 1;
+    c.xcd_remap = 1;
+    if (dtype != WK_F64) c.accumulate = WK_ACC_F64;
+  }
   // as the launcher uses it (a masked last tile where the windows run it)
   c.k_tile = std::min(c.k_tile, masked ? pow2_at_least(std::max(1, k)) : pow2_at_most(std::max(1, k)));
   return c;

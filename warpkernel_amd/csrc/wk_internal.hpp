@@ -75,6 +75,7 @@ void parallel_for(int64_t n, int64_t min_chunk, const std::function<void(int64_t
 struct DevLayout {
   int32_t variant = 1, W = 64;
   int32_t nrows = 0;      // rows of the product (ncols of A for the transpose)
+  int32_t ncols = 0;      // and its columns
   int32_t nznrows = 0, ngroups = 0;
   int64_t allocate_nz = 0;
   void *vals = nullptr;           // [allocate_nz] double or float
@@ -122,6 +123,15 @@ struct DevLayout {
   uint32_t *nd_pos = nullptr;      // [nd_off[ngroups] * 64] words, word-major, lane fastest
   uint32_t *nd_off = nullptr;      // [ngroups+1] first word of each group
   int32_t nd_max = 0;              // most entries in one group; 0: no node windows
+  // row sets (rowsets.hip): up to four neighbouring lanes of a group that read
+  // the same column at every step; built for WPK1 layouts whose sets hold two
+  // rows or more on average
+  void *rs_rec = nullptr;        // [rs_waves] four sets each: slots, rows, least columns
+  void *rs_cols = nullptr;       // their columns in the kernel's lane order: uint16 from
+                                 // each set's least column, or int32
+  void *rs_cols_kr = nullptr;    // the same in Kr numbering (int32)
+  bool rs_narrow = false;        // rs_cols holds uint16
+  int32_t rs_waves = 0;          // 0: no row sets
 };
 
 // Window positions fit the packed form up to this many entries per window.
@@ -200,6 +210,13 @@ void launch_scatter(const void *src, const uint32_t *index, void *dst, int64_t n
 // packed form (width 64, win_max <= kPackedWindow); otherwise leaves them null.
 // Then builds the node windows (D.nd_*) where the layout has them.
 void build_packed_positions(wk_engine *E, DevLayout &D, hipStream_t stream);
+// Builds the row sets (D.rs_*) of a layout, where they pay.
+void build_row_sets(wk_engine *E, DevLayout &D, hipStream_t stream);
+// k right-hand sides through the row sets.  prec: 0 FP64, 2 FP32 values with
+// FP64 accumulation.  Returns false, nothing launched, where the layout or the
+// vectors do not allow it.
+bool launch_rowsets(const DevLayout &D, int prec, int out, const SpmvArgs &a, int32_t k, int32_t remap,
+                    hipStream_t stream);
 void launch_fill_zero(void *p, int64_t bytes, hipStream_t stream);
 // Flags (int32) the column swap's check kernels write, one per block.
 constexpr int32_t kColFlags = 1024;
