@@ -39,8 +39,8 @@ void free_engine(wk_engine *E) {
 
 // Copies one host layout (and its padded values/columns) to the device.
 // vals/colind are the layout's own CSR; slot_of_nz (optional) replaces
-// reorder_rows as the device scatter map (the transpose is scattered from A's
-// CSR order).
+// reorder_rows as the map from A's CSR order to slots (the row sort and the
+// transpose, whose slots then take their CSR entries one by one).
 void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double *vals,
                    const int32_t *colind, int32_t dtype, bool kr, const uint32_t *slot_of_nz,
                    hipStream_t s) {
@@ -78,7 +78,15 @@ void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double 
     D.tpr = dev_upload(E, L.threads_per_row.data(), (int64_t)L.threads_per_row.size(), s);
     D.row_off = dev_upload(E, L.row_offset_warp.data(), (int64_t)L.row_offset_warp.size(), s);
   }
-  D.slot_of_nz = dev_upload(E, slot_of_nz ? slot_of_nz : L.reorder_rows.data(), L.nz, s);
+  std::vector<int32_t> src;
+  if (&D == &E->adj) {
+    src.assign((size_t)L.allocate_nz, -1);
+    for (int64_t i = 0; i < L.nz; i++) src[slot_of_nz[i]] = (int32_t)i;
+    D.src_of_slot = dev_upload(E, src.data(), (int64_t)src.size(), s);
+  } else {
+    D.slot_of_nz = dev_upload(E, slot_of_nz ? slot_of_nz : L.reorder_rows.data(), L.nz, s);
+    if (!slot_of_nz && lane_sources(L, src)) D.lane_src = dev_upload(E, src.data(), (int64_t)src.size(), s);
+  }
   hip_check(hipStreamSynchronize(s), "upload");
   if (L.W == 64) {
     // x windows: one key per slot, the entry's column or -1 for a pad
@@ -418,8 +426,7 @@ int wk_engine_update_values(wk_engine *E, const void *vals_dev, void *stream) {
     check_engine(E);
     if (!vals_dev && E->nnz) fail(WK_ERR_ARG, "vals_dev is NULL");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    launch_scatter_values(E->fwd, E->dtype, E->nnz, vals_dev, s);
-    if (E->has_adj) launch_scatter_values(E->adj, E->dtype, E->nnz, vals_dev, s);
+    launch_update_values(E, vals_dev, s);
   });
 }
 

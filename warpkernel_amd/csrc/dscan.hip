@@ -152,7 +152,8 @@ __global__ __launch_bounds__(kFillThreads) void fill_kernel(
     const int32_t *__restrict__ row_map_inv, const int64_t *__restrict__ wo,
     const uint32_t *__restrict__ aw, const uint32_t *__restrict__ tpr_a,
     const uint32_t *__restrict__ row_off, int32_t nznrows, T *__restrict__ pv,
-    int32_t *__restrict__ pc, int32_t *__restrict__ pkr, uint32_t *__restrict__ slot_of_nz) {
+    int32_t *__restrict__ pc, int32_t *__restrict__ pkr, uint32_t *__restrict__ slot_of_nz,
+    int2 *__restrict__ lane_src) {
   constexpr int PER = kFillSteps * 64 / kFillThreads;
   __shared__ int32_t first[64], count[64];        // each lane's first CSR entry, entries
   __shared__ T sv[64][kFillSteps + 1];            // odd row length: the turned reads spread
@@ -173,6 +174,7 @@ __global__ __launch_bounds__(kFillThreads) void fill_kernel(
     }
     first[tid] = rb;
     count[tid] = n;
+    lane_src[(int64_t)w * 64 + tid] = int2{rb, n};
   }
   __syncthreads();
   const int64_t base = wo[w];
@@ -491,7 +493,8 @@ void launch_fill(const DevLayout &D, const int32_t *rowptr, const int32_t *colin
   if (!D.ngroups) return;
   hipLaunchKernelGGL(fill_kernel<T>, dim3((uint32_t)D.ngroups), dim3(kFillThreads), 0, s, rowptr,
                      colind, vals, D.row_map, D.row_map_inv, D.warp_offsets, D.max_nz_rows, D.tpr,
-                     D.row_off, D.nznrows, static_cast<T *>(D.vals), D.cols, D.cols_kr, D.slot_of_nz);
+                     D.row_off, D.nznrows, static_cast<T *>(D.vals), D.cols, D.cols_kr, D.slot_of_nz,
+                     reinterpret_cast<int2 *>(D.lane_src));
   hip_check(hipGetLastError(), "fill");
 }
 
@@ -601,6 +604,7 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
   D.cols = dev_alloc<int32_t>(E, D.allocate_nz);
   D.cols_kr = kr ? dev_alloc<int32_t>(E, D.allocate_nz) : nullptr;
   D.slot_of_nz = dev_alloc<uint32_t>(E, nnz);
+  D.lane_src = dev_alloc<int32_t>(E, 128 * (int64_t)G);
   if (E->dtype == WK_F64) {
     D.vals = dev_alloc<double>(E, D.allocate_nz);
     launch_fill<double>(D, rowptr, colind, vals, s);

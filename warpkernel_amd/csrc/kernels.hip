@@ -615,14 +615,6 @@ __global__ void fill_zero_kernel(uint32_t *p, int64_t n) {
     p[i] = 0u;
 }
 
-template <class T>
-__global__ void scatter_kernel(const T *__restrict__ src, const uint32_t *__restrict__ slot,
-                               T *__restrict__ dst, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    dst[slot[i]] = src[i];
-}
-
 // thrust::scatter of the reference's _GPU helpers (warpkernel.hpp:459-502),
 // bounded: indices at or beyond dst_count are skipped.
 template <class T>
@@ -1729,22 +1721,6 @@ void launch_fill_zero(void *p, int64_t bytes, hipStream_t stream) {
   hipLaunchKernelGGL(fill_zero_kernel, dim3((uint32_t)blocks), dim3(256), 0, stream,
                      static_cast<uint32_t *>(p), n);
   hip_check(hipGetLastError(), "fill launch");
-}
-
-void launch_scatter_values(const DevLayout &D, int32_t dtype, int64_t nnz, const void *vals_csr,
-                           hipStream_t stream) {
-  if (nnz <= 0) return;
-  if (!D.slot_of_nz) fail(WK_ERR_STATE, "layout has no device scatter map");
-  const int64_t blocks = std::min<int64_t>((nnz + 255) / 256, 65536);
-  if (dtype == WK_F64)
-    hipLaunchKernelGGL(scatter_kernel<double>, dim3((uint32_t)blocks), dim3(256), 0, stream,
-                       static_cast<const double *>(vals_csr), D.slot_of_nz,
-                       static_cast<double *>(D.vals), nnz);
-  else
-    hipLaunchKernelGGL(scatter_kernel<float>, dim3((uint32_t)blocks), dim3(256), 0, stream,
-                       static_cast<const float *>(vals_csr), D.slot_of_nz,
-                       static_cast<float *>(D.vals), nnz);
-  hip_check(hipGetLastError(), "scatter launch");
 }
 
 void launch_scatter(const void *src, const uint32_t *index, void *dst, int64_t n, int64_t dst_count,

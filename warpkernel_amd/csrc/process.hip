@@ -1,0 +1,157 @@
+// process.hip -- new matrix values into an engine's layouts (wk_engine_update_values):
+// the reference's process step (warpkernel.hpp:379-398, 749-769) for values
+// alone, on the device.
+//
+// Layouts whose lanes hold runs of CSR entries (every forward layout without
+// the row sort): one block per group reads its rows' entries kSteps at a time,
+// turns them around in LDS and writes whole steps.  It streams 16 bytes per
+// FP64 entry, both ways in whole lines, with no index array.  (One thread per
+// entry writing through the CSR-to-slot map put 8 bytes into each 128-byte
+// line: hex elasticity 48^3, 27.4M entries, 305 us against 83.)  The
+// transposed layout reads the entry of each slot instead: indices and values
+// written in order, the 8-byte reads land on lines that the same group's other
+// steps read too (hex diffusion 48^3, both layouts 31 us as two scatters,
+// 24 here in one launch).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "spmv_device.hpp"
+#include "wk_internal.hpp"
+
+namespace wk {
+namespace {
+
+constexpr int kThreads = 256;
+constexpr int kSteps = 32;      // steps of a group turned at a time
+constexpr int kGatherPer = 8;   // slots per thread of the transposed layout
+
+struct UpdateArgs {
+  const void *src;                // CSR values
+  void *dst;                      // padded values
+  const int2 *lane_src;           // [ngroups * W] first CSR entry and entries of each lane
+  const int64_t *warp_offsets;
+  const uint32_t *max_nz_rows;
+  int32_t ngroups;
+  void *dst_t;                    // padded values of the transposed layout
+  const int32_t *src_of_slot;     // its slots' CSR entries, -1 for a pad
+  int64_t slots_t;
+  int32_t nblocks_t;              // blocks of the transposed layout
+};
+
+template <class T, int W>
+__device__ __forceinline__ void turn_group(const UpdateArgs &u, int32_t g) {
+  constexpr int PER = kSteps * W / kThreads;
+  __shared__ int2 ls[W];
+  __shared__ T tile[W][kSteps + 1];  // odd row length: the turned reads spread over the banks
+  const int32_t tid = threadIdx.x;
+  const T *src = static_cast<const T *>(u.src);
+  T *dst = static_cast<T *>(u.dst) + u.warp_offsets[g];
+  const int32_t len = (int32_t)u.max_nz_rows[g];
+  if (tid < W) ls[tid] = u.lane_src[(int64_t)g * W + tid];
+  __syncthreads();
+  for (int32_t i0 = 0; i0 < len; i0 += kSteps) {
+    T v[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+      const int2 s = ls[(tid + j * kThreads) / kSteps];
+      const int32_t i = i0 + tid % kSteps;
+      v[j] = i < s.y ? src[s.x + i] : T(0);
+    }
+#pragma unroll
+    for (int j = 0; j < PER; j++) tile[(tid + j * kThreads) / kSteps][tid % kSteps] = v[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+      const int32_t l = tid % W, t = (tid + j * kThreads) / W;
+      if (i0 + t < len) dst[l + (int64_t)W * (i0 + t)] = tile[l][t];
+    }
+    __syncthreads();
+  }
+}
+
+template <class T>
+__device__ __forceinline__ void gather_slots(const UpdateArgs &u, int32_t b) {
+  const T *src = static_cast<const T *>(u.src);
+  T *dst = static_cast<T *>(u.dst_t);
+  const int64_t s0 = (int64_t)b * (kThreads * kGatherPer) + threadIdx.x;
+  int32_t e[kGatherPer];
+#pragma unroll
+  for (int j = 0; j < kGatherPer; j++) {
+    const int64_t s = s0 + (int64_t)j * kThreads;
+    e[j] = s < u.slots_t ? u.src_of_slot[s] : -1;
+  }
+  T v[kGatherPer];
+#pragma unroll
+  for (int j = 0; j < kGatherPer; j++) v[j] = e[j] >= 0 ? src[e[j]] : T(0);
+#pragma unroll
+  for (int j = 0; j < kGatherPer; j++)
+    if (e[j] >= 0) dst[s0 + (int64_t)j * kThreads] = v[j];
+}
+
+// Blocks [0, ngroups): groups of the forward layout; then the transposed
+// layout's slots, each XCD a contiguous range of them.
+template <class T, int W>
+__global__ __launch_bounds__(kThreads) void update_kernel(UpdateArgs u) {
+  const int32_t b = blockIdx.x;
+  if (b < u.ngroups)
+    turn_group<T, W>(u, b);
+  else
+    gather_slots<T>(u, work_id(b - u.ngroups, u.nblocks_t, 1));
+}
+
+// Row-sorted layouts, whose lanes hold no runs: entry i to slot[i].
+template <class T>
+__global__ __launch_bounds__(kThreads) void scatter_kernel(const T *__restrict__ src,
+                                                           const uint32_t *__restrict__ slot,
+                                                           T *__restrict__ dst, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    dst[slot[i]] = src[i];
+}
+
+template <class T>
+void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
+  const DevLayout &D = E->fwd;
+  UpdateArgs u{};
+  u.src = vals;
+  if (D.lane_src) {
+    u.dst = D.vals;
+    u.lane_src = reinterpret_cast<const int2 *>(D.lane_src);
+    u.warp_offsets = D.warp_offsets;
+    u.max_nz_rows = D.max_nz_rows;
+    u.ngroups = D.ngroups;
+  } else {
+    if (!D.slot_of_nz) fail(WK_ERR_STATE, "layout has no device scatter map");
+    const int64_t blocks = std::min<int64_t>((E->nnz + kThreads - 1) / kThreads, 65536);
+    hipLaunchKernelGGL(scatter_kernel<T>, dim3((uint32_t)blocks), dim3(kThreads), 0, s,
+                       static_cast<const T *>(vals), D.slot_of_nz, static_cast<T *>(D.vals), E->nnz);
+    hip_check(hipGetLastError(), "scatter launch");
+  }
+  if (E->has_adj) {
+    u.dst_t = E->adj.vals;
+    u.src_of_slot = E->adj.src_of_slot;
+    u.slots_t = E->adj.allocate_nz;
+    u.nblocks_t = (int32_t)((u.slots_t + kThreads * kGatherPer - 1) / (kThreads * kGatherPer));
+  }
+  const int64_t blocks = (int64_t)u.ngroups + u.nblocks_t;
+  if (blocks > INT32_MAX) fail(WK_ERR_LIMIT, "grid too large");
+  if (blocks == 0) return;
+  if (D.W == 64)
+    hipLaunchKernelGGL((update_kernel<T, 64>), dim3((uint32_t)blocks), dim3(kThreads), 0, s, u);
+  else
+    hipLaunchKernelGGL((update_kernel<T, 32>), dim3((uint32_t)blocks), dim3(kThreads), 0, s, u);
+  hip_check(hipGetLastError(), "update launch");
+}
+
+}  // namespace
+
+void launch_update_values(const wk_engine *E, const void *vals_csr, hipStream_t stream) {
+  if (E->nnz <= 0) return;
+  if (E->dtype == WK_F64)
+    update_values<double>(E, vals_csr, stream);
+  else
+    update_values<float>(E, vals_csr, stream);
+}
+
+}  // namespace wk

@@ -245,6 +245,37 @@ void scan2(wk_layout &L, int32_t W, int32_t threshold, int32_t max_tpr, int32_t 
   });
 }
 
+bool lane_sources(const wk_layout &L, std::vector<int32_t> &src) {
+  src.assign((size_t)L.nwarps * L.W * 2, 0);
+  std::atomic<int64_t> entries{0};
+  std::atomic<bool> runs{true};
+  parallel_for(L.nwarps, 256, [&](int64_t w0, int64_t w1) {
+    int64_t n = 0;
+    bool ok = true;
+    for (int64_t w = w0; w < w1; w++) {
+      const uint32_t tpr = L.variant == 2 ? L.threads_per_row[w] : 1u, A = L.max_nz_rows[w];
+      const int64_t p0 = L.variant == 2 ? (int64_t)L.row_offset_warp[w] : w * L.W;
+      for (int32_t l = 0; l < L.W; l++) {
+        const int64_t p = p0 + l / tpr;
+        if (p >= L.nznrows) break;
+        const int32_t r = L.row_map[p];
+        const int64_t skip = (int64_t)(l % tpr) * A;
+        const int64_t left = (int64_t)L.rowptr[r + 1] - L.rowptr[r] - skip;
+        const int64_t len = std::max<int64_t>(0, std::min<int64_t>(left, A));
+        const int64_t e0 = L.rowptr[r] + skip;
+        for (int64_t i = 0; i < len; i++)
+          ok = ok && (int64_t)L.reorder_rows[e0 + i] == L.warp_offsets[w] + l + L.W * i;
+        if (len) src[(size_t)(w * L.W + l) * 2] = (int32_t)e0;
+        src[(size_t)(w * L.W + l) * 2 + 1] = (int32_t)len;
+        n += len;
+      }
+    }
+    entries += n;
+    if (!ok) runs = false;
+  });
+  return runs && entries == L.nz;
+}
+
 template <class T>
 void process_host(const wk_layout &L, const double *vals, const int32_t *colind, T *pvals,
                   int32_t *pcols) {

@@ -49,6 +49,10 @@ void scan1(wk_layout &L, int32_t W, int32_t nrows, int32_t ncols, int64_t nnz,
            const int32_t *rowptr);
 void scan2(wk_layout &L, int32_t W, int32_t threshold, int32_t max_tpr, int32_t nrows,
            int32_t ncols, int64_t nnz, const int32_t *rowptr);
+// The first CSR entry and the number of entries of every lane of every group
+// (two int32 each).  False where the layout's slots are not runs of CSR entries
+// in step order (arrays from elsewhere).
+bool lane_sources(const wk_layout &L, std::vector<int32_t> &src);
 // Host scatter through reorder_rows into zero-filled padded arrays (T = double or float).
 template <class T>
 void process_host(const wk_layout &L, const double *vals, const int32_t *colind, T *pvals,
@@ -87,7 +91,12 @@ struct DevLayout {
   uint32_t *max_nz_rows = nullptr;   // [ngroups]
   uint32_t *tpr = nullptr;           // [ngroups] (variant 2)
   uint32_t *row_off = nullptr;       // [ngroups+1] (variant 2)
-  uint32_t *slot_of_nz = nullptr;    // [nnz] CSR index -> padded slot (GPU process)
+  uint32_t *slot_of_nz = nullptr;    // [nnz] CSR index -> padded slot (forward layouts)
+  // GPU process: the first CSR entry and the entries of each lane of each group
+  // (forward layouts without the row sort), or every slot's CSR entry, -1 for a
+  // pad (transposed layouts)
+  int32_t *lane_src = nullptr;       // [ngroups * W * 2]
+  int32_t *src_of_slot = nullptr;    // [allocate_nz]
   std::vector<uint32_t> h_max_nz_rows;  // host copy (batch work partition)
   // x windows (stage_lds 3): each group's distinct columns, ascending, and per
   // slot the 16-bit position of its column in that list.  win_max = 0: none.
@@ -196,9 +205,9 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
                  const void *x, int64_t ldx, double *y, int64_t ldy, const double *b,
                  int64_t ldb, int32_t k, hipStream_t stream);
 
-// Zero-fill then scatter CSR values into the padded slots (GPU process).
-void launch_scatter_values(const DevLayout &D, int32_t dtype, int64_t nnz, const void *vals_csr,
-                           hipStream_t stream);
+// New CSR values (of the engine's type) into its forward and, where it has one,
+// transposed layout (GPU process).
+void launch_update_values(const wk_engine *E, const void *vals_csr, hipStream_t stream);
 void launch_stream_read(const void *p, int64_t bytes, uint32_t *sink, hipStream_t stream);
 void launch_gather_ceiling(const DevLayout &D, const wk_launch &cfg, const double *x, double *y,
                            hipStream_t stream);
