@@ -2,7 +2,9 @@
 32 steps the fill turns at a time, column spans on both sides of the 262,144
 bits of the window bitmap, pads, duplicate columns and split rows.  Every array
 equals the host-scanned engine's (whole numbers and copied values: no tolerance)."""
+import gc
 import sys
+import weakref
 
 import numpy as np
 import pytest
@@ -64,3 +66,60 @@ def test_device_scan_equals_host_scan(name, variant, dtype):
         assert np.array_equal(a, b), (which, a.size, b.size)
     host.close()
     dev.close()
+
+
+def test_device_scanned_engine_is_freed_when_dropped():
+    """Without the garbage collector; its layout keeps it alive while held."""
+    say("[gpu] device-scanned engine lifetime")
+    m = matrix(130, [3, 1, 7], 60, 1)
+    csr = [torch.from_numpy(a).cuda() for a in (m.rowptr, m.colind, m.vals)]
+    rows = structure(64).scan(m.nnz, m.nrows, m.vals, m.rowptr, m.colind).row_map
+    gc.disable()
+    try:
+        eng = engine.from_device(*csr)
+        ref = weakref.ref(eng)
+        assert eng.kernel is eng.kernel or eng.kernel.nz == m.nnz
+        assert np.array_equal(eng.kernel.row_map, rows) and eng.kernel.row_map is eng.kernel.row_map
+        layout = eng.kernel
+        del eng
+        assert ref() is not None and layout.nrows == m.nrows
+        assert np.array_equal(layout.row_map_inv[layout.row_map], np.arange(m.nrows))
+        del layout
+        assert ref() is None
+        eng = engine.from_device(*csr)
+        eng.close()
+        assert eng.kernel.nz == m.nnz  # the scalars outlive the device arrays
+    finally:
+        gc.enable()
+
+
+def test_rebuilt_engines_reuse_device_blocks():
+    """Engines rebuilt in place keep their results while blocks change hands
+    (another engine alive, launches in flight when one is destroyed), and the
+    device memory held afterwards is bounded."""
+    say("[gpu] rebuilt engines")
+    free0 = torch.cuda.mem_get_info()[0]
+    mats = [fe.hex_elastic_3d(n) for n in (24, 20, 25)]
+    csr = [[torch.from_numpy(a).cuda() for a in (m.rowptr, m.colind, m.vals)] for m in mats]
+    xs = [torch.from_numpy(fe.uniform_x(m.ncols, seed=i)).cuda() for i, m in enumerate(mats)]
+    first = []
+    for m, c, x in zip(mats, csr, xs):
+        y = torch.full((m.nrows,), float("nan"), dtype=torch.float64, device="cuda")
+        eng = engine.from_device(*c)
+        eng.launch(x, y)
+        first.append(y.clone())
+    kept = engine.from_device(*csr[0])  # stays alive while the others come and go
+    for rep in range(12):
+        i = rep % 3
+        ys = torch.full((mats[i].nrows,), float("nan"), dtype=torch.float64, device="cuda")
+        eng = engine.from_device(*csr[i])
+        eng.launch(xs[i], ys)
+        eng.close()  # the product may still be running
+        yk = torch.full((mats[0].nrows,), float("nan"), dtype=torch.float64, device="cuda")
+        kept.launch(xs[0], yk)
+        assert torch.equal(ys, first[i]) and torch.equal(yk, first[0]), rep
+    kept.close()
+    del csr, xs, first, ys, yk
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    assert free0 - torch.cuda.mem_get_info()[0] < (3 << 30)  # 2 GiB kept at most

@@ -21,6 +21,7 @@ Differences, all deliberate:
 from __future__ import annotations
 
 import ctypes as C
+import weakref
 
 import numpy as np
 
@@ -209,7 +210,7 @@ class engine:
                  adjoint: bool = False, rowsort: bool = False, stream=None):
         if k._h is None:
             raise ValueError("structure has not been scanned")
-        self.kernel = k
+        self._structure = k
         self.dtype = {"f64": capi.WK_F64, "f32": capi.WK_F32}[dtype]
         A = np.ascontiguousarray(A, dtype=np.float64)
         colinds = np.ascontiguousarray(colinds, dtype=np.int32)
@@ -237,6 +238,7 @@ class engine:
                 raise ValueError("rowptr/colind must be contiguous int32 and vals float64 device tensors")
         self = cls.__new__(cls)
         self._h = None
+        self._structure, self._layout, self._arrays, self._info = None, None, {}, None
         self.dtype = {"f64": capi.WK_F64, "f32": capi.WK_F32}[dtype]
         nrows = rowptr.numel() - 1
         nnz = colind.numel()
@@ -249,10 +251,31 @@ class engine:
                                             self.dtype, capi.WK_ENGINE_KR if kr else 0,
                                             _stream(stream), C.byref(h)))
         self._h = h
-        self.kernel = _EngineLayout(self)
+        self._info = capi.LayoutInfo()
+        check(lib().wk_engine_get_info(h, C.byref(self._info)))
         self.nrows, self.ncols, self.nz = nrows, ncols, nnz
         self.has_kr, self.has_adjoint = kr, False
         return self
+
+    @property
+    def kernel(self):
+        """The scanned structure, or the layout scanned on the device.  The latter
+        refers to its engine and the engine only weakly to it: as a cycle they
+        waited for the garbage collector, and a program that rebuilds its
+        engine piled up hundreds of them on the device (hex elasticity 40^3,
+        300 rebuilds: 9 to 12 ms each on average, single ones over a second,
+        against 1.3 ms freed at once)."""
+        if self._structure is not None:
+            return self._structure
+        layout = self._layout() if self._layout is not None else None
+        if layout is None:
+            layout = _EngineLayout(self)
+            self._layout = weakref.ref(layout)
+        return layout
+
+    @kernel.setter
+    def kernel(self, k):
+        self._structure = k
 
     def download(self, which: int) -> np.ndarray:
         """One device array of the forward layout (WK_ROW_MAP .. WK_ROW_OFFSET_WARP,
@@ -464,7 +487,7 @@ class engine:
 
 class _EngineLayout:
     """The layout of an engine scanned on the device: structure's scalars, and
-    its arrays downloaded on first use."""
+    its arrays downloaded on first use (kept with the engine)."""
 
     _ARRAYS = {"row_map": capi.WK_ROW_MAP, "row_map_inv": capi.WK_ROW_MAP_INV,
                "reorder_rows": capi.WK_REORDER_ROWS, "warp_offsets": capi.WK_WARP_OFFSETS,
@@ -473,9 +496,7 @@ class _EngineLayout:
 
     def __init__(self, eng: "engine"):
         self._eng = eng
-        info = capi.LayoutInfo()
-        check(lib().wk_engine_get_info(eng._h, C.byref(info)))
-        self.info = info
+        info = self.info = eng._info
         self.variant, self.group_width = info.variant, info.group_width
         self.nrows, self.ncols, self.nznrows = info.nrows, info.ncols, info.nznrows
         self.nz, self.allocate_nz, self.nwarps = info.nz, info.allocate_nz, info.nwarps
@@ -483,9 +504,10 @@ class _EngineLayout:
 
     def __getattr__(self, name):
         if name in _EngineLayout._ARRAYS:
-            a = self._eng.download(_EngineLayout._ARRAYS[name])
-            setattr(self, name, a)
-            return a
+            kept = self._eng._arrays
+            if name not in kept:
+                kept[name] = self._eng.download(_EngineLayout._ARRAYS[name])
+            return kept[name]
         raise AttributeError(name)
 
 

@@ -8,6 +8,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/warpkernel_c.h"
@@ -173,7 +174,7 @@ struct wk_engine {
   int32_t *d_colind = nullptr;
   int32_t *d_tile_row = nullptr;    // dvals tile -> first row
   int32_t *d_rowind = nullptr;      // row of every CSR entry (dvals)
-  std::vector<void *> owned;        // every hipMalloc of this engine
+  std::vector<std::pair<void *, size_t>> owned;  // every device block of this engine and its size
   int device = 0;
   std::mutex cfg_mu;                // guards launch_cfg
   std::map<int64_t, wk_launch> launch_cfg;  // (op << 32 | k) -> configuration
@@ -286,13 +287,19 @@ int guarded(F &&f) {
   }
 }
 
-// Device allocations owned (and freed) by an engine.
+// Device blocks of the current device: bytes is raised to the block's size.
+// Blocks go back with block_give, which may keep them for the next engine;
+// nothing on the device may still use them.
+void *block_take(size_t &bytes);
+void block_give(int device, void *p, size_t bytes) noexcept;
+
+// Device allocations owned (and given back) by an engine.
 template <class T>
 T *dev_alloc(wk_engine *E, int64_t count) {
   if (count <= 0) return nullptr;
-  void *p = nullptr;
-  hip_check(hipMalloc(&p, sizeof(T) * (size_t)count), "hipMalloc");
-  E->owned.push_back(p);
+  size_t bytes = sizeof(T) * (size_t)count;
+  void *p = block_take(bytes);
+  E->owned.push_back({p, bytes});
   return static_cast<T *>(p);
 }
 
