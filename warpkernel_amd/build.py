@@ -29,7 +29,7 @@ HIP_FLAGS = [
 ]
 HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-pthread"]
 
-LIB_SOURCES = ["kernels.hip", "rowsets.hip", "process.hip", "batch.hip", "dscan.hip", "assembly.hip", "colinds.hip", "noalloc.hip", "capi.cpp",
+LIB_SOURCES = ["kernels.hip", "rowsets.hip", "process.hip", "deltas.hip", "batch.hip", "dscan.hip", "assembly.hip", "colinds.hip", "noalloc.hip", "capi.cpp",
                "scan.cpp", "tune.cpp", "io.cpp"]
 
 

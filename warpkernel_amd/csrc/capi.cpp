@@ -144,6 +144,28 @@ void free_engine(wk_engine *E) {
   delete E;
 }
 
+}  // namespace
+
+void build_compact_columns(wk_engine *E, DevLayout &D, uint32_t *scratch, hipStream_t stream) {
+  const size_t G = (size_t)std::max(D.ngroups, 0);
+  // downloaded: starts, spans and a word more, fits; then the groups' first words
+  const size_t words = 2 * G + (G + 1) + G;
+  uint64_t *starts = reinterpret_cast<uint64_t *>(scratch);
+  uint32_t *span = scratch + 2 * G, *fits = span + G + 1;
+  std::vector<uint32_t> off;
+  const bool sets = row_sets_begin(D, starts, span, stream);
+  const bool offsets = deltas_begin(E, D, off, fits, scratch + words, stream);
+  if (!sets && !offsets) return;
+  std::vector<uint64_t> h((words + 1) / 2);
+  hip_check(hipMemcpyAsync(h.data(), scratch, 4 * words, hipMemcpyDeviceToHost, stream), "compact columns");
+  hip_check(hipStreamSynchronize(stream), "compact columns");
+  const uint32_t *hw = reinterpret_cast<const uint32_t *>(h.data());
+  if (offsets) deltas_finish(D, hw + 3 * G + 1);
+  if (sets) row_sets_finish(E, D, starts, span, h.data(), hw + 2 * G, stream);
+}
+
+namespace {
+
 // Copies one host layout (and its padded values/columns) to the device.
 // vals/colind are the layout's own CSR; slot_of_nz (optional) replaces
 // reorder_rows as the map from A's CSR order to slots (the row sort and the
@@ -219,7 +241,7 @@ void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double 
         hip_check(hipStreamSynchronize(s), "upload");
       }
       build_packed_positions(E, D, s);
-      build_row_sets(E, D, s);
+      build_compact_columns(E, D, dev_alloc<uint32_t>(E, compact_words(D.ngroups)), s);
     } else {
       D.win_max = 0;
     }

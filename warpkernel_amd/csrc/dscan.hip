@@ -588,8 +588,10 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
   D.h_max_nz_rows = A;
   D.warp_offsets = dev_upload(E, wo.data(), (int64_t)wo.size(), s);
   D.max_nz_rows = dev_upload(E, A.data(), G, s);
+  std::vector<uint32_t> tpr, roff;  // (uploads: alive until the next wait)
   if (variant == 2) {
-    std::vector<uint32_t> tpr((size_t)G), roff((size_t)G + 1, 0);
+    tpr.resize((size_t)G);
+    roff.assign((size_t)G + 1, 0);
     for (int32_t w = 0; w < G; w++) {
       tpr[w] = 64u / rows_nominal[w];
       roff[w + 1] = roff[w] + rows_actual[w];
@@ -597,14 +599,14 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
     roff[G] = (uint32_t)nrows;  // sentinel (hpp:716)
     D.tpr = dev_upload(E, tpr.data(), G, s);
     D.row_off = dev_upload(E, roff.data(), G + 1, s);
-    hip_check(hipStreamSynchronize(s), "upload");
   }
 
   // 4. padded arrays and the CSR -> slot map
   D.cols = dev_alloc<int32_t>(E, D.allocate_nz);
   D.cols_kr = kr ? dev_alloc<int32_t>(E, D.allocate_nz) : nullptr;
-  D.slot_of_nz = dev_alloc<uint32_t>(E, nnz);
-  D.lane_src = dev_alloc<int32_t>(E, 128 * (int64_t)G);
+  const int64_t even = nnz + (nnz & 1);  // (first entry, entries) pairs follow the map
+  D.slot_of_nz = dev_alloc<uint32_t>(E, even + 128 * (int64_t)G);
+  D.lane_src = reinterpret_cast<int32_t *>(D.slot_of_nz + even);
   if (E->dtype == WK_F64) {
     D.vals = dev_alloc<double>(E, D.allocate_nz);
     launch_fill<double>(D, rowptr, colind, vals, s);
@@ -612,13 +614,14 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
     D.vals = dev_alloc<float>(E, D.allocate_nz);
     launch_fill<float>(D, rowptr, colind, vals, s);
   }
-  hip_check(hipStreamSynchronize(s), "device scan");
+  if (!G) hip_check(hipStreamSynchronize(s), "device scan");  // (else: the window counts' download)
 
   // 5. x windows, when every group fits
   if (G) {
     WinBuild wb{rowptr, D.row_map, D.row_map_inv, D.cols, D.warp_offsets, D.max_nz_rows,
                 D.tpr, D.row_off, nznrows};
-    int32_t *dcount = dev_alloc<int32_t>(E, 2 * (int64_t)G);
+    // read and written before build_compact_columns takes it
+    int32_t *dcount = dev_alloc<int32_t>(E, compact_words(G));
     hipLaunchKernelGGL(window_count_kernel, dim3((uint32_t)G), dim3(kWinThreads), 0, s, wb, dcount,
                        dcount + G);
     hip_check(hipGetLastError(), "window count");
@@ -648,7 +651,7 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
       D.win_max = most;
       D.win_total = off[G];
       build_packed_positions(E, D, s);
-      build_row_sets(E, D, s);
+      build_compact_columns(E, D, reinterpret_cast<uint32_t *>(dcount), s);
     }
   }
 

@@ -378,25 +378,22 @@ bool launch_rowsets(const DevLayout &D, int prec, int out, const SpmvArgs &a0, i
   return true;
 }
 
-void build_row_sets(wk_engine *E, DevLayout &D, hipStream_t stream) {
+bool row_sets_begin(DevLayout &D, uint64_t *starts, uint32_t *span, hipStream_t stream) {
   D.rs_waves = 0;
   const int32_t G = D.ngroups;
-  if (D.variant != 1 || D.W != 64 || D.win_max <= 0 || G <= 0 || !D.cols) return;
+  if (D.variant != 1 || D.W != 64 || D.win_max <= 0 || G <= 0 || !D.cols) return false;
   for (int32_t g = 0; g < G; g++)
-    if (set_chunks((int32_t)D.h_max_nz_rows[g]) > kMaxChunks) return;
+    if (set_chunks((int32_t)D.h_max_nz_rows[g]) > kMaxChunks) return false;
   const int64_t blocks = ((int64_t)G + kBuildWaves - 1) / kBuildWaves;
-  // set starts, then spans; after the download the space of the spans and one
-  // more word takes the groups' first waves (few allocations and copies: an
-  // engine scanned on the device is built in about a millisecond)
-  uint64_t *starts = dev_alloc<uint64_t>(E, G + ((int64_t)G + 2) / 2);
-  uint32_t *span = reinterpret_cast<uint32_t *>(starts + G);
   hipLaunchKernelGGL(row_set_kernel, dim3((uint32_t)blocks), dim3(kBuildWaves * 64), 0, stream, D.cols,
                      D.warp_offsets, D.max_nz_rows, G, starts, span);
   hip_check(hipGetLastError(), "row set launch");
-  std::vector<uint64_t> hs((size_t)G + ((size_t)G + 1) / 2);
-  hip_check(hipMemcpyAsync(hs.data(), starts, 12 * (size_t)G, hipMemcpyDeviceToHost, stream), "row sets");
-  hip_check(hipStreamSynchronize(stream), "row sets");
-  const uint32_t *hw = reinterpret_cast<const uint32_t *>(hs.data() + G);
+  return true;
+}
+
+void row_sets_finish(wk_engine *E, DevLayout &D, const uint64_t *starts, uint32_t *span, const uint64_t *hs,
+                     const uint32_t *hw, hipStream_t stream) {
+  const int32_t G = D.ngroups;
   std::vector<uint32_t> woff((size_t)G + 1, 0);
   int64_t sets = 0, waves = 0;
   uint32_t widest = 0;

@@ -197,6 +197,59 @@ __device__ __forceinline__ void stream_tail(typename P::Acc (&acc)[KT], const ty
     }
 }
 
+// One group with 16-bit column offsets (deltas.hip): column = row + offset, or
+// column 0 for kDeltaZero; a word holds a lane's next four steps.  Batches of U
+// steps, all loads of a batch before its first use; the last one partial.
+constexpr int32_t kDeltaZero = -32768;
+
+template <class P, int U>
+__device__ __forceinline__ typename P::Acc delta_steps(const typename P::V *vp, const uint2 *wp,
+                                                       const typename P::X *xb, int64_t ldx, uint32_t len,
+                                                       int32_t row) {
+  using V = typename P::V;
+  using X = typename P::X;
+  static_assert(U % 4 == 0, "whole words");
+  auto column = [&](const uint2 &w, int u) {
+    const uint32_t h = u < 2 ? w.x : w.y;
+    const int32_t d = u & 1 ? (int32_t)h >> 16 : (int32_t)(h << 16) >> 16;
+    return d == kDeltaZero ? 0 : row + d;
+  };
+  typename P::Acc acc;
+  P::init(acc);  // every slot by fma onto -0 (see PF64::init)
+  uint32_t i = 0;
+  for (; i + U <= len; i += U) {
+    uint2 w[U / 4];
+    V v[U];
+#pragma unroll
+    for (int q = 0; q < U / 4; q++) w[q] = wp[(int64_t)(i / 4 + q) * 64];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = __builtin_nontemporal_load(vp + (int64_t)(i + u) * 64);
+    X xv[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) xv[u] = xb[(int64_t)column(w[u / 4], u % 4) * ldx];
+#pragma unroll
+    for (int u = 0; u < U; u++) P::step(acc, v[u], xv[u]);
+  }
+  if (i < len) {
+    uint2 w[U / 4];
+    V v[U];
+#pragma unroll
+    for (int q = 0; q < U / 4; q++)
+      if (i + 4 * q < len) w[q] = wp[(int64_t)(i / 4 + q) * 64];
+#pragma unroll
+    for (int u = 0; u < U - 1; u++)
+      if (i + u < len) v[u] = __builtin_nontemporal_load(vp + (int64_t)(i + u) * 64);
+    X xv[U];
+#pragma unroll
+    for (int u = 0; u < U - 1; u++)
+      if (i + u < len) xv[u] = xb[(int64_t)column(w[u / 4], u % 4) * ldx];
+#pragma unroll
+    for (int u = 0; u < U - 1; u++)
+      if (i + u < len) P::step(acc, v[u], xv[u]);
+  }
+  return acc;
+}
+
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 template <class P, int U>

@@ -133,7 +133,7 @@ std::vector<wk_launch> candidates(const DevLayout &D, int32_t dtype, const wk_la
 
 }  // namespace
 
-wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k) {
+wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr) {
   wk_launch c;
   wk_launch_default(&c);
   bool masked = false;  // k-tiles may exceed k (windowed multi-RHS)
@@ -160,7 +160,25 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k) {
                               (D.variant == 2 && k >= 8 && reuse >= 2.5) ||
                               (dtype == WK_F64 && D.variant == 1 && k >= 4 && reuse >= 2.0 &&
                                mean_len < 20.0 && D.ngroups >= 4096));
-  if (k == 1 && windows) {
+  // large layouts keep windows that are reused most (hex diffusion 100^3, 16,098
+  // groups, 3.4 slots per entry, 49.9 us against 52.3 by offsets; but 72^3, 6,079
+  // groups, 22.4 against 21.4, and FP32 100^3 33.3 against 29.9)
+  const bool keep_windows =
+      windows && D.ngroups >= 8192 && (reuse >= 4.5 || (dtype == WK_F64 && mean_len >= 20.0));
+  if (k == 1 && !kr && D.dl_words && win_ok && D.nd_max == 0 && !keep_windows) {
+    // 16-bit column offsets (deltas.hip).  P1 tets 96^3 30.4 -> 27.8 us (FP32
+    // 23.9 -> 18.8), 60^3 9.5 -> 7.5; large layouts without the remap (96^3 27.8
+    // against 28.8, FP32 18.8 against 21.6; 60^3 7.6 against 7.4).  Ahead of the
+    // windows too, most on small layouts, where filling them is a serial step (2D
+    // Laplacian 27^2 2.3 us against 3.3, hex diffusion 22^3 4.0 against 5.0, 48^3
+    // 7.1 against 7.4) and on WPK2's short groups (threshold 5: tets 96^3 32.9
+    // against 39.7 direct, 2D Laplacian 600^2 8.8 against 15.7, hex diffusion
+    // 48^3 10.5 against 17.5)
+    c.stage_lds = 0;
+    c.unroll = 8;  // (the steps in flight: launch_deltas)
+    c.waves_per_block = 2;
+    c.xcd_remap = D.variant == 2 || D.ngroups < 8192;
+  } else if (k == 1 && windows) {
     // 10 bytes per slot, x from the group's window in LDS; one wave per
     // block, a contiguous range of groups per XCD, and 16-step batches for
     // long groups (hex elasticity 64^3: 99.3 us against 104 with 8-step
@@ -381,7 +399,7 @@ wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k) {
     auto it = E->launch_cfg.find(cfg_key(op, k));
     if (it != E->launch_cfg.end()) return it->second;
   }
-  return heuristic_launch(layout_for(E, op), E->dtype, k);
+  return heuristic_launch(layout_for(E, op), E->dtype, k, op == WK_OP_RUN_X);
 }
 
 }  // namespace wk

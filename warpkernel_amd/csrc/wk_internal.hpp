@@ -133,6 +133,11 @@ struct DevLayout {
   uint32_t *nd_pos = nullptr;      // [nd_off[ngroups] * 64] words, word-major, lane fastest
   uint32_t *nd_off = nullptr;      // [ngroups+1] first word of each group
   int32_t nd_max = 0;              // most entries in one group; 0: no node windows
+  // 16-bit column offsets (deltas.hip): short rows, every column within 32,767
+  // of its row or 0, windows that do not pay; per group ceil(len/4) words of 64
+  // lanes x 8 bytes
+  uint32_t *dl_words = nullptr;  // [dl_off[ngroups] * 128]
+  uint32_t *dl_off = nullptr;    // [ngroups+1]
   // row sets (rowsets.hip): up to four neighbouring lanes of a group that read
   // the same column at every step; built for WPK1 layouts whose sets hold two
   // rows or more on average
@@ -220,13 +225,29 @@ void launch_scatter(const void *src, const uint32_t *index, void *dst, int64_t n
 // packed form (width 64, win_max <= kPackedWindow); otherwise leaves them null.
 // Then builds the node windows (D.nd_*) where the layout has them.
 void build_packed_positions(wk_engine *E, DevLayout &D, hipStream_t stream);
-// Builds the row sets (D.rs_*) of a layout, where they pay.
-void build_row_sets(wk_engine *E, DevLayout &D, hipStream_t stream);
+// Builds the row sets (D.rs_*) and the 16-bit column offsets (D.dl_*) of a
+// layout that has them: both checks on the device, then one download.
+// scratch: compact_words(ngroups) words on the device, the engine's.
+inline int64_t compact_words(int32_t ngroups) { return 5 * (int64_t)ngroups + 2; }
+void build_compact_columns(wk_engine *E, DevLayout &D, uint32_t *scratch, hipStream_t stream);
+// Row sets: starts [ngroups] and span [ngroups + 1] on the device; finish takes
+// the downloaded first ngroups of each and reuses span.
+bool row_sets_begin(DevLayout &D, uint64_t *starts, uint32_t *span, hipStream_t stream);
+void row_sets_finish(wk_engine *E, DevLayout &D, const uint64_t *starts, uint32_t *span, const uint64_t *hs,
+                     const uint32_t *hw, hipStream_t stream);
+// Offsets: fits [ngroups] on the device, downloaded for finish; off stays alive
+// until then, dev_off [ngroups + 1] as long as the engine.
+bool deltas_begin(wk_engine *E, DevLayout &D, std::vector<uint32_t> &off, uint32_t *fits, uint32_t *dev_off,
+                  hipStream_t stream);
+void deltas_finish(DevLayout &D, const uint32_t *fits);
 // k right-hand sides through the row sets.  prec: 0 FP64, 2 FP32 values with
 // FP64 accumulation.  Returns false, nothing launched, where the layout or the
 // vectors do not allow it.
 bool launch_rowsets(const DevLayout &D, int prec, int out, const SpmvArgs &a, int32_t k, int32_t remap,
                     hipStream_t stream);
+// One right-hand side through them (wpb waves per block, unroll 8 or 16).  False, nothing launched, where the layout has none.
+bool launch_deltas(const DevLayout &D, int prec, int out, const SpmvArgs &a, int wpb, int unroll, int32_t remap,
+                   hipStream_t stream);
 void launch_fill_zero(void *p, int64_t bytes, hipStream_t stream);
 // Flags (int32) the column swap's check kernels write, one per block.
 constexpr int32_t kColFlags = 1024;
@@ -259,7 +280,7 @@ int64_t dvals_tile_size();
 // The configuration an engine uses for (op, k) when the caller passes none:
 // the tuned one if any, else a choice from the layout.
 wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k);
-wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k);
+wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr);
 
 // WPK2's group split (warpkernel.hpp:633-691) over the longest row of each
 // W-row group of sorted rows (aw0); nzr = non-empty rows.  Outputs per
