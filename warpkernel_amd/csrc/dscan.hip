@@ -49,7 +49,17 @@ __global__ __launch_bounds__(256) void csr_check_kernel(const int32_t *__restric
     if (len < 0) bad |= 2;
     m = max(m, len);
   }
-  for (int64_t e = t0; e < nnz; e += stride)
+  // four columns a load where colind allows it (hex elasticity 40^3, 16M columns,
+  // 32 -> 16 us)
+  const int64_t n4 = ((uintptr_t)colind & 15) == 0 ? nnz / 4 : 0;
+  const int4 *c4 = reinterpret_cast<const int4 *>(colind);
+#pragma unroll 4
+  for (int64_t e = t0; e < n4; e += stride) {
+    const int4 c = c4[e];
+    const uint32_t most = max(max((uint32_t)c.x, (uint32_t)c.y), max((uint32_t)c.z, (uint32_t)c.w));
+    if (most >= (uint32_t)ncols) bad |= 4;
+  }
+  for (int64_t e = 4 * n4 + t0; e < nnz; e += stride)
     if ((uint32_t)colind[e] >= (uint32_t)ncols) bad |= 4;
   if (t0 == 0 && (rowptr[0] != 0 || (int64_t)rowptr[nrows] != nnz)) bad |= 1;
   red_max[threadIdx.x] = m;
@@ -126,11 +136,13 @@ __global__ __launch_bounds__(64) void place_kernel(const int32_t *__restrict__ r
   }
 }
 
-// aw[g] = length of sorted row 64 g, the longest of group g
+// aw[g] = length of sorted row 64 g, the longest of group g; aw[ngroups] that of
+// the last nonempty row, the shortest
 __global__ __launch_bounds__(256) void group_len_kernel(const uint32_t *__restrict__ slen,
-                                                        int32_t ngroups, uint32_t *__restrict__ aw) {
+                                                        int32_t ngroups, int32_t nznrows,
+                                                        uint32_t *__restrict__ aw) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g < ngroups) aw[g] = slen[g * 64];
+  if (g <= ngroups) aw[g] = slen[g < ngroups ? g * 64 : nznrows - 1];
 }
 
 // One block per (sub-)group w: lane l holds chunk l % tpr of sorted row
@@ -219,16 +231,23 @@ __global__ __launch_bounds__(kFillThreads) void fill_kernel(
 
 // ---------------------------------------------------------------- x windows
 // The windows of build_windows (scan.cpp), built on the device, one block per
-// group: the distinct slot keys (the entry's column, -1 for a pad) are counted
-// (pass 1), then written with each slot's position among them (pass 2).  Where
-// the group's columns span at most kWinBits (every banded ordering) the keys
-// set bits of an LDS bitmap, and a key's position is the number of bits below
-// its own: the words' running counts plus one popcount.  Wider groups sort
-// their keys in LDS.  (Sorting every group took 1.01 + 1.38 ms on hex elasticity
-// 40^3, 3,231 groups of 5,184 slots; the bitmap BIT_US.)  Groups of more than
-// kWinSlots slots are not handled here: the engine then has no windows.
+// group: the distinct slot keys (the entry's column, -1 for a pad) in ascending
+// order, and each slot's position among them.
+//
+// Where the group's columns span at most kWinBits (every banded ordering) they are
+// read once, into registers, set bits of an LDS bitmap, and a key's position is the
+// number of bits below its own: the words' running counts plus one popcount
+// (window_kernel; spans of at most kBandBits first, with 12 KB of LDS and so the
+// occupancy of the registers, then the others).  Wider groups sort their keys in
+// LDS (window_sort_kernel).  The keys go to a stash, since where they belong is
+// known only when every group has been counted; window_place_kernel copies them
+// there.  Hex elasticity 40^3, 3,231 groups of 5,184 slots: sorting every group,
+// once to count and once to write, took 1.01 + 1.38 ms; the bitmap in two such
+// passes, which read the columns five times, 88 + 117 us; 52 + 24 us here, and 7 to place.  Groups of
+// more than kWinSlots slots are not handled: the engine then has no windows.
 constexpr int32_t kWinSlots = 8192;
 constexpr int32_t kWinBits = kWinSlots * 32;  // the bitmap takes the sort's LDS
+constexpr int32_t kBandBits = 65536;
 constexpr int kWinThreads = 256;
 
 struct WinBuild {
@@ -288,18 +307,8 @@ __device__ void sort_group_keys(const WinBuild &b, int32_t g, int32_t S, int32_t
 struct Span {
   int32_t lo, hi, pad;
 };
-__device__ Span group_span(const WinBuild &b, int64_t base, int32_t S, const int32_t *lane_n, int32_t *red) {
+__device__ Span block_span(int32_t lo, int32_t hi, int32_t pad, int32_t *red) {
   const int32_t tid = threadIdx.x;
-  int32_t lo = INT32_MAX, hi = -1, pad = 0;
-  for (int32_t t = tid; t < S; t += kWinThreads) {
-    if ((t >> 6) < lane_n[t & 63]) {
-      const int32_t c = b.cols[base + t];
-      lo = min(lo, c);
-      hi = max(hi, c);
-    } else {
-      pad = 1;
-    }
-  }
   for (int o = 32; o > 0; o >>= 1) {
     lo = min(lo, __shfl_xor(lo, o));
     hi = max(hi, __shfl_xor(hi, o));
@@ -320,160 +329,179 @@ __device__ Span group_span(const WinBuild &b, int64_t base, int32_t S, const int
   return {lo, hi, pad};
 }
 
-// Sets the bit of every entry's column in bits[0, words) (bit 0: column lo).
-__device__ void group_bits(const WinBuild &b, int64_t base, int32_t S, const int32_t *lane_n, int32_t lo,
-                           int32_t words, uint32_t *bits) {
-  for (int32_t t = threadIdx.x; t < words; t += kWinThreads) bits[t] = 0;
-  __syncthreads();
-  for (int32_t t = threadIdx.x; t < S; t += kWinThreads)
-    if ((t >> 6) < lane_n[t & 63]) {
-      const uint32_t k = (uint32_t)(b.cols[base + t] - lo);
-      atomicOr(&bits[k >> 5], 1u << (k & 31));
-    }
-  __syncthreads();
-}
-
-// Inclusive sum of every thread's c over the block (part: kWinThreads ints).
-__device__ int32_t block_scan(int32_t c, int32_t *part) {
-  const int32_t tid = threadIdx.x;
-  part[tid] = c;
-  __syncthreads();
-  for (int o = 1; o < kWinThreads; o <<= 1) {
-    const int32_t v = tid >= o ? part[tid - o] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
+// Inclusive sum of every thread's c over the block; total: the whole sum (red:
+// kWinThreads / 64 ints, free again after the next barrier).
+__device__ int32_t block_scan(int32_t c, int32_t *red, int32_t &total) {
+  const int32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int32_t v = __shfl_up(c, o);
+    if (lane >= o) c += v;
   }
-  return part[tid];
+  if (lane == 63) red[wave] = c;
+  __syncthreads();
+  total = 0;
+  for (int w = 0; w < kWinThreads / 64; w++) {
+    if (w < wave) c += red[w];
+    total += red[w];
+  }
+  return c;
 }
 
-// count[g]: distinct keys, or -1; words[g]: bitmap words of the group, or
-// INT32_MAX where its keys have to be sorted.
-__global__ __launch_bounds__(kWinThreads) void window_count_kernel(WinBuild b, int32_t *count, int32_t *nwords) {
-  __shared__ int32_t keys[kWinSlots];
+// count[g]: distinct keys, -1 where they are more than kMaxWindow, kWide where the
+// columns span more than BITS.  stash[g][stride]: the keys.  R: slots of a thread,
+// kWinThreads R at least the longest group's.  The kernel for more than kBandBits
+// takes only the groups that the one before it has marked.
+constexpr int32_t kWide = -2;
+template <int R, int BITS>
+__global__ __launch_bounds__(kWinThreads) void window_kernel(WinBuild b, int32_t stride,
+                                                             int32_t *__restrict__ count,
+                                                             int32_t *__restrict__ stash,
+                                                             uint16_t *__restrict__ win_idx) {
+  __shared__ uint32_t bits[BITS / 32];
+  __shared__ uint16_t below[BITS / 32];  // bits in the words before
   __shared__ int32_t lane_n[64];
-  __shared__ int32_t part[kWinThreads];
+  __shared__ int32_t red[32];
   const int32_t g = blockIdx.x;
-  const int64_t S64 = (int64_t)b.aw[g] * 64;
-  if (S64 > kWinSlots) {
-    if (threadIdx.x == 0) {
-      count[g] = -1;
-      nwords[g] = 0;
+  const int32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (BITS > kBandBits && count[g] != kWide) return;
+  const int32_t A = (int32_t)b.aw[g];
+  const int64_t base = b.wo[g] + tid;
+  int32_t c[R];
+#pragma unroll
+  for (int j = 0; j < R; j++) c[j] = wave + 4 * j < A ? b.cols[base + kWinThreads * j] : 0;
+  lane_entries(b, g, lane_n);
+  const int32_t n = lane_n[lane];
+  int32_t lo = INT32_MAX, hi = -1, pad = 0;
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    const int32_t i = wave + 4 * j;
+    if (i < n) {
+      lo = min(lo, c[j]);
+      hi = max(hi, c[j]);
+    } else if (i < A) {
+      pad = 1;
     }
+  }
+  const Span sp = block_span(lo, hi, pad, red);
+  if (sp.hi - sp.lo >= BITS) {
+    if (tid == 0) count[g] = kWide;
     return;
   }
-  const int32_t S = (int32_t)S64;
-  const int64_t base = b.wo[g];
-  lane_entries(b, g, lane_n);
-  const Span sp = group_span(b, base, S, lane_n, part);
-  int32_t c = 0;
-  if (sp.hi - sp.lo < kWinBits) {
-    const int32_t words = (sp.hi - sp.lo + 32) >> 5;
-    uint32_t *bits = reinterpret_cast<uint32_t *>(keys);
-    group_bits(b, base, S, lane_n, sp.lo, words, bits);
-    for (int32_t t = threadIdx.x; t < words; t += kWinThreads) c += __popc(bits[t]);
-    if (threadIdx.x == 0) c += sp.pad;
-  } else {
-    int32_t N = 0;  // the keys in LDS: S rounded up to a power of two
-    sort_group_keys(b, g, S, keys, lane_n, N);
-    for (int32_t t = threadIdx.x; t < N; t += kWinThreads)
-      c += keys[t] != INT32_MAX && (t == 0 || keys[t] != keys[t - 1]);
-  }
-  const int32_t total = block_scan(c, part);
-  if (threadIdx.x == kWinThreads - 1) {
-    count[g] = total > kMaxWindow ? -1 : total;
-    nwords[g] = sp.hi - sp.lo < kWinBits ? (sp.hi - sp.lo + 32) >> 5 : INT32_MAX;
-  }
-}
-
-// WIDE: some group's keys have to be sorted (dynamic LDS for kWinSlots keys);
-// otherwise 6 bytes of dynamic LDS for each of nw bitmap words.
-template <bool WIDE>
-__global__ __launch_bounds__(kWinThreads) void window_write_kernel(WinBuild b, const uint32_t *off,
-                                                                   int32_t *win_cols,
-                                                                   int32_t *win_cols_kr,
-                                                                   uint16_t *win_idx, int32_t nw) {
-  extern __shared__ int32_t keys[];
-  uint16_t *below = reinterpret_cast<uint16_t *>(keys + nw);  // bits in the words before
-  __shared__ int32_t uniq[WIDE ? kMaxWindow : 1];
-  __shared__ int32_t lane_n[64];
-  __shared__ int32_t part[kWinThreads];
-  const int32_t g = blockIdx.x;
-  const int32_t tid = threadIdx.x;
-  const int32_t S = (int32_t)b.aw[g] * 64;  // at most kWinSlots: the host builds windows only then
-  const int64_t base = b.wo[g];
-  const uint32_t w0 = off[g];
-  lane_entries(b, g, lane_n);
-  const Span sp = group_span(b, base, S, lane_n, part);
-  if (!WIDE || sp.hi - sp.lo < kWinBits) {
-    const int32_t words = (sp.hi - sp.lo + 32) >> 5;
-    uint32_t *bits = reinterpret_cast<uint32_t *>(keys);
-    group_bits(b, base, S, lane_n, sp.lo, words, bits);
-    const int32_t per = (words + kWinThreads - 1) / kWinThreads;
-    const int32_t t0 = min(words, tid * per), t1 = min(words, t0 + per);
-    int32_t c = 0;
-    for (int32_t t = t0; t < t1; t++) c += __popc(bits[t]);
-    int32_t rank = block_scan(c, part) - c + sp.pad;  // a pad's key is the first
-    if (tid == 0 && sp.pad) {
-      win_cols[w0] = 0;
-      if (win_cols_kr) win_cols_kr[w0] = 0;
+  const int32_t words = sp.hi < sp.lo ? 0 : (sp.hi - sp.lo + 32) >> 5;
+  for (int32_t t = tid; t < words; t += kWinThreads) bits[t] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < R; j++)
+    if (wave + 4 * j < n) {
+      const uint32_t k = (uint32_t)(c[j] - sp.lo), bit = 1u << (k & 31);
+      // most columns come from several slots: only the first pay the atomic
+      if (!(bits[k >> 5] & bit)) atomicOr(&bits[k >> 5], bit);
     }
-    for (int32_t t = t0; t < t1; t++) {
-      below[t] = (uint16_t)rank;
-      for (uint32_t m = bits[t]; m; m &= m - 1) {
-        const int32_t k = sp.lo + 32 * t + (__ffs((int)m) - 1);
-        win_cols[w0 + rank] = k;
-        if (win_cols_kr) win_cols_kr[w0 + rank] = b.row_map_inv[k];
-        rank++;
-      }
-    }
-    __syncthreads();
-    for (int32_t t = tid; t < S; t += kWinThreads) {
+  __syncthreads();
+  const int32_t per = ((words + kWinThreads - 1) / kWinThreads) | 1;  // odd: no bank conflicts
+  const int32_t t0 = min(words, tid * per), t1 = min(words, t0 + per);
+  int32_t sum = 0, total;
+  for (int32_t t = t0; t < t1; t++) sum += __popc(bits[t]);
+  int32_t rank = block_scan(sum, red, total) - sum + sp.pad;  // a pad's key is the first
+  total += sp.pad;
+  if (tid == 0) count[g] = total > kMaxWindow ? -1 : total;
+  if (total > kMaxWindow) return;
+  int32_t *keys = stash + (int64_t)g * stride;
+  if (tid == 0 && sp.pad) keys[0] = -1;
+  for (int32_t t = t0; t < t1; t++) {
+    below[t] = (uint16_t)rank;
+    for (uint32_t m = bits[t]; m; m &= m - 1) keys[rank++] = sp.lo + 32 * t + (__ffs((int)m) - 1);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    const int32_t i = wave + 4 * j;
+    if (i < A) {
       int32_t p = 0;
-      if ((t >> 6) < lane_n[t & 63]) {
-        const uint32_t k = (uint32_t)(b.cols[base + t] - sp.lo);
+      if (i < n) {
+        const uint32_t k = (uint32_t)(c[j] - sp.lo);
         p = below[k >> 5] + __popc(bits[k >> 5] & ((1u << (k & 31)) - 1u));
       }
-      win_idx[base + t] = (uint16_t)p;
-    }
-    return;
-  }
-  if constexpr (WIDE) {
-    int32_t N = 0;
-    sort_group_keys(b, g, S, keys, lane_n, N);
-    // ranks of the distinct keys: each thread counts a contiguous chunk of the
-    // sorted keys, then an inclusive scan of the chunk counts
-    const int32_t per = N / kWinThreads > 0 ? N / kWinThreads : 1;
-    const int32_t t0 = min(N, tid * per), t1 = min(N, t0 + per);
-    int32_t c = 0;
-    for (int32_t t = t0; t < t1; t++) c += keys[t] != INT32_MAX && (t == 0 || keys[t] != keys[t - 1]);
-    int32_t rank = block_scan(c, part) - c;
-    for (int32_t t = t0; t < t1; t++) {
-      const int32_t k = keys[t];
-      if (k != INT32_MAX && (t == 0 || k != keys[t - 1])) {
-        uniq[rank] = k;
-        win_cols[w0 + rank] = k < 0 ? 0 : k;
-        if (win_cols_kr) win_cols_kr[w0 + rank] = k < 0 ? 0 : b.row_map_inv[k];
-        rank++;
-      }
-    }
-    __syncthreads();
-    // each slot's position among the distinct keys (ascending; a pad's key -1,
-    // when present, is the first)
-    const int32_t n = part[kWinThreads - 1];
-    for (int32_t t = tid; t < S; t += kWinThreads) {
-      const int32_t key = (t >> 6) < lane_n[t & 63] ? b.cols[base + t] : -1;
-      int32_t lo = 0, hi = n;
-      while (lo < hi) {
-        const int32_t mid = (lo + hi) >> 1;
-        if (uniq[mid] < key)
-          lo = mid + 1;
-        else
-          hi = mid;
-      }
-      win_idx[base + t] = (uint16_t)lo;
+      win_idx[base + kWinThreads * j] = (uint16_t)p;
     }
   }
+}
+
+// The groups that are still marked.
+__global__ __launch_bounds__(kWinThreads) void window_sort_kernel(WinBuild b, int32_t stride,
+                                                                  int32_t *__restrict__ count,
+                                                                  int32_t *__restrict__ stash,
+                                                                  uint16_t *__restrict__ win_idx) {
+  __shared__ int32_t keys[kWinSlots];
+  __shared__ int32_t uniq[kMaxWindow];
+  __shared__ int32_t lane_n[64];
+  __shared__ int32_t red[32];
+  const int32_t g = blockIdx.x;
+  const int32_t tid = threadIdx.x;
+  if (count[g] != kWide) return;
+  const int32_t S = (int32_t)b.aw[g] * 64;  // at most kWinSlots
+  const int64_t base = b.wo[g];
+  lane_entries(b, g, lane_n);
+  int32_t N = 0, n;  // the keys in LDS: S rounded up to a power of two
+  sort_group_keys(b, g, S, keys, lane_n, N);
+  // ranks of the distinct keys: each thread counts a contiguous chunk of the
+  // sorted keys, then an inclusive scan of the chunk counts
+  const int32_t per = N / kWinThreads > 0 ? N / kWinThreads : 1;
+  const int32_t t0 = min(N, tid * per), t1 = min(N, t0 + per);
+  int32_t c = 0;
+  for (int32_t t = t0; t < t1; t++) c += keys[t] != INT32_MAX && (t == 0 || keys[t] != keys[t - 1]);
+  int32_t rank = block_scan(c, red, n) - c;
+  if (tid == 0) count[g] = n > kMaxWindow ? -1 : n;
+  if (n > kMaxWindow) return;
+  for (int32_t t = t0; t < t1; t++) {
+    const int32_t k = keys[t];
+    if (k != INT32_MAX && (t == 0 || k != keys[t - 1])) {
+      uniq[rank] = k;
+      stash[(int64_t)g * stride + rank] = k;
+      rank++;
+    }
+  }
+  __syncthreads();
+  // each slot's position among the distinct keys (ascending; a pad's key -1,
+  // when present, is the first)
+  for (int32_t t = tid; t < S; t += kWinThreads) {
+    const int32_t key = (t >> 6) < lane_n[t & 63] ? b.cols[base + t] : -1;
+    int32_t lo = 0, hi = n;
+    while (lo < hi) {
+      const int32_t mid = (lo + hi) >> 1;
+      if (uniq[mid] < key)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    win_idx[base + t] = (uint16_t)lo;
+  }
+}
+
+__global__ __launch_bounds__(kWinThreads) void window_place_kernel(const int32_t *__restrict__ stash, int32_t stride,
+                                                                   const uint32_t *__restrict__ off,
+                                                                   const int32_t *__restrict__ row_map_inv,
+                                                                   int32_t *__restrict__ win_cols,
+                                                                   int32_t *__restrict__ win_cols_kr) {
+  const int32_t g = blockIdx.x;
+  const uint32_t w0 = off[g], n = off[g + 1] - w0;
+  for (uint32_t t = threadIdx.x; t < n; t += kWinThreads) {
+    const int32_t k = stash[(int64_t)g * stride + t];
+    win_cols[w0 + t] = k < 0 ? 0 : k;
+    if (win_cols_kr) win_cols_kr[w0 + t] = k < 0 ? 0 : row_map_inv[k];
+  }
+}
+
+template <int R>
+void launch_windows(const WinBuild &b, int32_t ngroups, int32_t ncols, int32_t stride, int32_t *count,
+                    int32_t *stash, uint16_t *win_idx, hipStream_t s) {
+  const dim3 grid((uint32_t)ngroups), block(kWinThreads);
+  hipLaunchKernelGGL((window_kernel<R, kBandBits>), grid, block, 0, s, b, stride, count, stash, win_idx);
+  if (ncols > kBandBits)
+    hipLaunchKernelGGL((window_kernel<R, kWinBits>), grid, block, 0, s, b, stride, count, stash, win_idx);
+  if (ncols > kWinBits)
+    hipLaunchKernelGGL(window_sort_kernel, grid, block, 0, s, b, stride, count, stash, win_idx);
+  hip_check(hipGetLastError(), "windows");
 }
 
 template <class T>
@@ -497,6 +525,24 @@ void launch_fill(const DevLayout &D, const int32_t *rowptr, const int32_t *colin
                      reinterpret_cast<int2 *>(D.lane_src));
   hip_check(hipGetLastError(), "fill");
 }
+
+// Device memory for a part of the scan, given back at its end; idle: nothing uses
+// it any more (on an error its kernels may still run).
+struct Stash {
+  int device;
+  size_t bytes;
+  int32_t *p;
+  bool idle = false;
+  Stash(int dev, size_t n)
+      : device(dev), bytes(n), p(n ? static_cast<int32_t *>(block_take(bytes)) : nullptr) {}
+  ~Stash() {
+    if (!p) return;
+    if (!idle) (void)hipDeviceSynchronize();
+    block_give(device, p, bytes);
+  }
+  Stash(const Stash &) = delete;
+  Stash &operator=(const Stash &) = delete;
+};
 
 // Scan + process of one device CSR into E->fwd.
 void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_tpr, bool kr,
@@ -567,12 +613,13 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
   std::vector<uint32_t> aw0;
   uint32_t shortest = 0;
   if (G0) {
-    uint32_t *daw = dev_alloc<uint32_t>(E, G0);
-    hipLaunchKernelGGL(group_len_kernel, dim3((uint32_t)((G0 + 255) / 256)), dim3(256), 0, s, slen,
-                       G0, daw);
+    uint32_t *daw = dev_alloc<uint32_t>(E, (int64_t)G0 + 1);
+    hipLaunchKernelGGL(group_len_kernel, dim3((uint32_t)(G0 / 256 + 1)), dim3(256), 0, s, slen,
+                       G0, nznrows, daw);
     hip_check(hipGetLastError(), "group_len");
-    aw0 = download(daw, G0, s);
-    shortest = download(slen + nznrows - 1, 1, s)[0];
+    aw0 = download(daw, (int64_t)G0 + 1, s);
+    shortest = aw0.back();
+    aw0.pop_back();
   }
   std::vector<uint32_t> A, rows_nominal, rows_actual;
   if (variant == 2)
@@ -617,21 +664,30 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
   if (!G) hip_check(hipStreamSynchronize(s), "device scan");  // (else: the window counts' download)
 
   // 5. x windows, when every group fits
-  if (G) {
+  const uint32_t longest = G ? *std::max_element(A.begin(), A.end()) : 0;
+  if (G && (int64_t)longest * 64 <= kWinSlots) {
     WinBuild wb{rowptr, D.row_map, D.row_map_inv, D.cols, D.warp_offsets, D.max_nz_rows,
                 D.tpr, D.row_off, nznrows};
-    // read and written before build_compact_columns takes it
-    int32_t *dcount = dev_alloc<int32_t>(E, compact_words(G));
-    hipLaunchKernelGGL(window_count_kernel, dim3((uint32_t)G), dim3(kWinThreads), 0, s, wb, dcount,
-                       dcount + G);
-    hip_check(hipGetLastError(), "window count");
-    const std::vector<int32_t> cnt = download(dcount, 2 * (int64_t)G, s);
+    const int32_t stride = std::min((int32_t)longest * 64, kMaxWindow);
+    const int64_t keys = (int64_t)stride * G;
+    const bool small = keys <= 65536;  // an allocation less
+    // (counts: read and written before build_compact_columns takes them)
+    int32_t *dcount = dev_alloc<int32_t>(E, compact_words(G) + (small ? keys : 0));
+    Stash taken(E->device, small ? 0 : sizeof(int32_t) * (size_t)keys);
+    int32_t *stash = small ? dcount + compact_words(G) : taken.p;
+    uint16_t *idx = dev_alloc<uint16_t>(E, D.allocate_nz);
+    const auto launch = longest <= 16   ? launch_windows<4>
+                        : longest <= 32 ? launch_windows<8>
+                        : longest <= 96 ? launch_windows<24>
+                                        : launch_windows<32>;
+    launch(wb, G, ncols, stride, dcount, stash, idx, s);
+    const std::vector<int32_t> cnt = download(dcount, G, s);
+    taken.idle = true;
     bool fits = true;
     std::vector<uint32_t> off((size_t)G + 1, 0);
-    int32_t most = 0, words = 0;
+    int32_t most = 0;
     for (int32_t g = 0; g < G && fits; g++) {
       if (cnt[g] < 0) fits = false;
-      words = std::max(words, cnt[(size_t)G + g]);
       off[g + 1] = off[g] + (uint32_t)std::max(cnt[g], 0);
       most = std::max(most, cnt[g]);
     }
@@ -639,19 +695,20 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
       D.win_off = dev_upload(E, off.data(), (int64_t)off.size(), s);
       D.win_cols = dev_alloc<int32_t>(E, off[G]);
       D.win_cols_kr = kr ? dev_alloc<int32_t>(E, off[G]) : nullptr;
-      D.win_idx = dev_alloc<uint16_t>(E, D.allocate_nz);
-      if (words > kWinSlots)  // the words of the groups that have a bitmap, or the sort's keys
-        hipLaunchKernelGGL(window_write_kernel<true>, dim3((uint32_t)G), dim3(kWinThreads), 6 * kWinSlots, s,
-                           wb, D.win_off, D.win_cols, D.win_cols_kr, D.win_idx, kWinSlots);
-      else
-        hipLaunchKernelGGL(window_write_kernel<false>, dim3((uint32_t)G), dim3(kWinThreads),
-                           6 * (size_t)words, s, wb, D.win_off, D.win_cols, D.win_cols_kr, D.win_idx, words);
-      hip_check(hipGetLastError(), "window write");
-      hip_check(hipStreamSynchronize(s), "window write");
+      D.win_idx = idx;
+      taken.idle = false;
+      hipLaunchKernelGGL(window_place_kernel, dim3((uint32_t)G), dim3(kWinThreads), 0, s, stash, stride, D.win_off,
+                         D.row_map_inv, D.win_cols, D.win_cols_kr);
+      hip_check(hipGetLastError(), "window place");
       D.win_max = most;
       D.win_total = off[G];
       build_packed_positions(E, D, s);
+      hip_check(hipStreamSynchronize(s), "window place");
+      taken.idle = true;
       build_compact_columns(E, D, reinterpret_cast<uint32_t *>(dcount), s);
+    } else {
+      block_give(E->device, E->owned.back().first, E->owned.back().second);  // idx
+      E->owned.pop_back();
     }
   }
 

@@ -1543,38 +1543,40 @@ void launch_stream_read(const void *p, int64_t bytes, uint32_t *sink, hipStream_
   hip_check(hipGetLastError(), "stream read launch");
 }
 
-// One wave per group: lane l packs its positions of steps 12b .. 12b+11 into
-// four words, three 10-bit fields each (steps past the group's length are 0).
+// One block per group, its waves on every fourth batch: lane l packs its
+// positions of steps 12b .. 12b+11 into four words, three 10-bit fields each
+// (steps past the group's length are 0).  (A wave per group left most of the chip
+// idle: hex elasticity 40^3, 3,231 groups, 31 -> 10 us.)
 __global__ __launch_bounds__(256) void pack_positions_kernel(const uint16_t *__restrict__ idx,
                                                              const int64_t *__restrict__ warp_offsets,
                                                              const uint32_t *__restrict__ max_nz_rows,
                                                              const uint32_t *__restrict__ pk_off,
-                                                             int32_t ngroups, u32x4 *__restrict__ out) {
-  const int32_t g = (int32_t)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+                                                             u32x4 *__restrict__ out) {
+  const int32_t g = (int32_t)blockIdx.x;
   const int32_t lane = threadIdx.x & 63;
-  if (g >= ngroups) return;
-  const int64_t base = warp_offsets[g];
+  const int64_t base = warp_offsets[g] + lane;
   const uint32_t len = max_nz_rows[g];
   const uint32_t nbat = pk_off[g + 1] - pk_off[g];
-  for (uint32_t b = 0; b < nbat; b++) {
-    uint32_t w[4] = {0u, 0u, 0u, 0u};
+  for (uint32_t b = threadIdx.x >> 6; b < nbat; b += 4) {
+    uint32_t p[12], w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int u = 0; u < 12; u++) {
-      const uint32_t i = b * 12 + u;
-      if (i < len) w[u / 3] |= (uint32_t)idx[base + lane + 64 * (int64_t)i] << (10 * (u % 3));
-    }
+    for (int u = 0; u < 12; u++) p[u] = idx[base + 64 * (int64_t)min(b * 12 + u, len - 1)];
+#pragma unroll
+    for (int u = 0; u < 12; u++) w[u / 3] |= (b * 12 + u < len ? p[u] : 0u) << (10 * (u % 3));
     out[((int64_t)pk_off[g] + b) * 64 + lane] = u32x4{w[0], w[1], w[2], w[3]};
   }
 }
 
-// Node windows from the windows of a layout, one wave per group.  Pass 1
-// (nd_pos null) checks that every triple of a lane's steps reads either a node
-// (three consecutive window positions holding columns 3n, 3n+1, 3n+2) or one
-// position three times, and counts the group's entries: per window position
-// in order, a node entry where a node starts there, then a constant entry
-// where some triple reads that position three times.  It writes the count, or
-// kNdNone when the group does not fit.  Pass 2 (every group fits) writes the
-// entries and each lane's entry indices, three 10-bit fields to a word.
+// Node windows from the windows of a layout, one block per group, its waves on
+// every fourth triple of steps.  Pass 1 (nd_pos null) checks that every triple of
+// a lane's steps reads either a node (three consecutive window positions holding
+// columns 3n, 3n+1, 3n+2) or one position three times, and counts the group's
+// entries: per window position in order, a node entry where a node starts there,
+// then a constant entry where some triple reads that position three times.  It
+// writes the count, or kNdNone when the group does not fit.  Pass 2 (every group
+// fits) writes the entries and each lane's entry indices, three 10-bit fields to a
+// word.  (A wave per group, its loads one triple at a time: hex elasticity 40^3,
+// 3,231 groups, 38 + 25 us; 21 + 15 here.)
 constexpr uint32_t kNdNone = 0xffffffffu;
 constexpr int kNdWaves = 4;
 
@@ -1582,90 +1584,91 @@ __global__ __launch_bounds__(kNdWaves * 64) void node_window_kernel(
     const uint16_t *__restrict__ idx, const int64_t *__restrict__ warp_offsets,
     const uint32_t *__restrict__ max_nz_rows, const uint32_t *__restrict__ win_off,
     const int32_t *__restrict__ win_cols, const int32_t *__restrict__ win_cols_kr,
-    int32_t ngroups, uint32_t *__restrict__ cnt, const uint32_t *__restrict__ nd_off,
+    uint32_t *__restrict__ cnt, const uint32_t *__restrict__ nd_off,
     int32_t *__restrict__ nd_cols, int32_t *__restrict__ nd_cols_kr,
     uint32_t *__restrict__ nd_pos) {
   // per window position: bit 0 a node starts here, bit 1 read as a constant triple
-  __shared__ uint8_t kind[kNdWaves][kPackedWindow];
+  __shared__ uint8_t kind[kPackedWindow];
   // per window position: the entry of the node starting there, of the constant
-  __shared__ uint16_t entry_of[kNdWaves][kPackedWindow][2];
-  const int32_t wib = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int32_t g = (int32_t)blockIdx.x * kNdWaves + wib;
-  const bool live = g < ngroups;
-  uint32_t n = 0, len = 0, w0 = 0;
-  int64_t base = 0;
-  if (live) {
-    w0 = win_off[g];
-    n = win_off[g + 1] - w0;  // at most kPackedWindow (packed windows only)
-    len = max_nz_rows[g];
-    base = warp_offsets[g];
-  }
-  uint8_t *kd = kind[wib];
+  __shared__ uint16_t entry_of[kPackedWindow][2];
+  __shared__ uint32_t some_bad;
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int32_t g = (int32_t)blockIdx.x;
+  const uint32_t w0 = win_off[g], n = win_off[g + 1] - w0;  // n at most kPackedWindow (packed windows only)
+  const uint32_t len = max_nz_rows[g];                      // a multiple of 3 (build_node_windows)
+  const uint16_t *ip = idx + warp_offsets[g] + lane;
   const int32_t *wc = win_cols + w0;
-  for (uint32_t p = (uint32_t)lane; p < n; p += 64) {
+  if (threadIdx.x == 0) some_bad = 0;
+  for (uint32_t p = threadIdx.x; p < n; p += kNdWaves * 64) {
     const int32_t c = wc[p];
     const bool st = c % 3 == 0 && p + 2 < n && wc[p + 1] == c + 1 && wc[p + 2] == c + 2;
-    kd[p] = st ? 1 : 0;
+    kind[p] = st ? 1 : 0;
   }
   __syncthreads();
-  bool bad = live && len % 3 != 0;
-  if (live && len % 3 == 0) {
-    for (uint32_t t = 0; t < len; t += 3) {
-      const int64_t s = base + lane + 64 * (int64_t)t;
-      const uint32_t p0 = idx[s], p1 = idx[s + 64], p2 = idx[s + 128];
-      if (p1 == p0 + 1 && p2 == p0 + 2 && (kd[p0] & 1)) continue;
-      if (p0 == p1 && p1 == p2)
-        kd[p0] |= 2;  // lanes only set bit 1 here: concurrent writes agree
+  bool bad = false;
+  constexpr uint32_t T = 7;  // triples in flight; past the end the last one again
+  for (uint32_t t0 = 3 * wave; t0 < len; t0 += 3 * kNdWaves * T) {
+    uint32_t p[T][3];
+#pragma unroll
+    for (uint32_t u = 0; u < T; u++)
+      for (uint32_t d = 0; d < 3; d++) p[u][d] = ip[64 * (int64_t)(min(t0 + 3 * kNdWaves * u, len - 3) + d)];
+#pragma unroll
+    for (uint32_t u = 0; u < T; u++) {
+      if (p[u][1] == p[u][0] + 1 && p[u][2] == p[u][0] + 2 && (kind[p[u][0]] & 1)) continue;
+      if (p[u][0] == p[u][1] && p[u][1] == p[u][2])
+        kind[p[u][0]] |= 2;  // only bit 1 is set here: concurrent writes agree
       else
         bad = true;
     }
   }
+  if (__ballot(bad) && lane == 0) some_bad = 1;
   __syncthreads();
+  // entries: each wave those of a quarter of the positions, after counting the ones before
   uint32_t total = 0;
   const uint64_t below = (1ull << lane) - 1;
-  for (uint32_t p0 = 0; p0 < n; p0 += 64) {
-    const uint32_t p = p0 + (uint32_t)lane;
-    const uint32_t k = p < n ? kd[p] : 0u;
+  constexpr uint32_t Q = kPackedWindow / kNdWaves;
+  const uint32_t p_end = min(n, nd_pos ? (wave + 1) * Q : n);
+  for (uint32_t p0 = 0; p0 < p_end; p0 += 64) {
+    const uint32_t p = p0 + lane;
+    const uint32_t k = p < n ? kind[p] : 0u;
     const uint64_t ms = __ballot(k & 1u), mc = __ballot((k >> 1) & 1u);
-    const uint32_t r = total + (uint32_t)__popcll(ms & below) + (uint32_t)__popcll(mc & below);
-    if (k & 1u) {
-      entry_of[wib][p][0] = (uint16_t)r;
-      if (nd_pos) nd_cols[w0 + r] = wc[p];
-      if (nd_pos && nd_cols_kr)
-        for (uint32_t d = 0; d < 3; d++) nd_cols_kr[3 * ((int64_t)w0 + r) + d] = win_cols_kr[w0 + p + d];
-    }
-    if (k & 2u) {
-      const uint32_t rc = r + (k & 1u);
-      entry_of[wib][p][1] = (uint16_t)rc;
-      if (nd_pos) nd_cols[w0 + rc] = -wc[p] - 1;
-      if (nd_pos && nd_cols_kr)
-        for (uint32_t d = 0; d < 3; d++) nd_cols_kr[3 * ((int64_t)w0 + rc) + d] = win_cols_kr[w0 + p];
+    if (nd_pos && p0 >= wave * Q) {
+      const uint32_t r = total + (uint32_t)__popcll(ms & below) + (uint32_t)__popcll(mc & below);
+      if (k & 1u) {
+        entry_of[p][0] = (uint16_t)r;
+        nd_cols[w0 + r] = wc[p];
+        if (nd_cols_kr)
+          for (uint32_t d = 0; d < 3; d++) nd_cols_kr[3 * ((int64_t)w0 + r) + d] = win_cols_kr[w0 + p + d];
+      }
+      if (k & 2u) {
+        const uint32_t rc = r + (k & 1u);
+        entry_of[p][1] = (uint16_t)rc;
+        nd_cols[w0 + rc] = -wc[p] - 1;
+        if (nd_cols_kr)
+          for (uint32_t d = 0; d < 3; d++) nd_cols_kr[3 * ((int64_t)w0 + rc) + d] = win_cols_kr[w0 + p];
+      }
     }
     total += (uint32_t)__popcll(ms) + (uint32_t)__popcll(mc);
   }
-  bad = __ballot(bad) != 0 || total > n;
-  __syncthreads();
-  if (!live) return;
   if (!nd_pos) {
-    if (lane == 0) cnt[g] = bad ? kNdNone : total;
+    if (threadIdx.x == 0) cnt[g] = some_bad || total > n ? kNdNone : total;
     return;
   }
+  __syncthreads();
   // pass 2: each lane's entry index per triple of steps, 27 steps to 3 words
-  const uint32_t nblk = (len + 26) / 27;
+  const uint32_t nwords = 3 * ((len + 26) / 27);
   uint32_t *dst = nd_pos + (int64_t)nd_off[g] * 64 + lane;
-  for (uint32_t bk = 0; bk < nblk; bk++)
-    for (uint32_t q = 0; q < 3; q++) {
-      uint32_t word = 0;
-      for (uint32_t f = 0; f < 3; f++) {
-        const uint32_t t = bk * 27 + q * 9 + f * 3;
-        if (t < len) {
-          const int64_t s = base + lane + 64 * (int64_t)t;
-          const uint32_t p0 = idx[s], p1 = idx[s + 64];
-          word |= (uint32_t)entry_of[wib][p0][p1 == p0 + 1 ? 0 : 1] << (10 * f);
-        }
-      }
-      dst[((int64_t)bk * 3 + q) * 64] = word;
-    }
+  for (uint32_t q = wave; q < nwords; q += kNdWaves) {
+    uint32_t p[3][2], word = 0;
+#pragma unroll
+    for (uint32_t f = 0; f < 3; f++)
+      for (uint32_t d = 0; d < 2; d++) p[f][d] = ip[64 * (int64_t)(min(9 * q + 3 * f, len - 3) + d)];
+#pragma unroll
+    for (uint32_t f = 0; f < 3; f++)
+      if (9 * q + 3 * f < len)
+        word |= (uint32_t)entry_of[p[f][0]][p[f][1] == p[f][0] + 1 ? 0 : 1] << (10 * f);
+    dst[(int64_t)q * 64] = word;
+  }
 }
 
 static void build_node_windows(wk_engine *E, DevLayout &D, hipStream_t stream) {
@@ -1679,11 +1682,9 @@ static void build_node_windows(wk_engine *E, DevLayout &D, hipStream_t stream) {
   if (!D.win_pk || !D.win_cols || !D.win_off || D.win_total <= 0 || G <= 0) return;
   for (int32_t g = 0; g < G; g++)
     if (D.h_max_nz_rows[g] % 3) return;
-  const int64_t blocks = ((int64_t)G + kNdWaves - 1) / kNdWaves;
   uint32_t *cnt = dev_alloc<uint32_t>(E, G);
-  hipLaunchKernelGGL(node_window_kernel, dim3((uint32_t)blocks), dim3(kNdWaves * 64), 0, stream,
-                     D.win_idx, D.warp_offsets, D.max_nz_rows, D.win_off, D.win_cols, nullptr, G,
-                     cnt, nullptr, nullptr, nullptr, nullptr);
+  hipLaunchKernelGGL(node_window_kernel, dim3((uint32_t)G), dim3(kNdWaves * 64), 0, stream,
+                     D.win_idx, D.warp_offsets, D.max_nz_rows, D.win_off, D.win_cols, nullptr, cnt, nullptr, nullptr, nullptr, nullptr);
   hip_check(hipGetLastError(), "node window launch");
   std::vector<uint32_t> h((size_t)G);
   hip_check(hipMemcpyAsync(h.data(), cnt, sizeof(uint32_t) * (size_t)G, hipMemcpyDeviceToHost, stream),
@@ -1702,9 +1703,9 @@ static void build_node_windows(wk_engine *E, DevLayout &D, hipStream_t stream) {
   D.nd_pos = dev_alloc<uint32_t>(E, (int64_t)off.back() * 64);
   D.nd_cols = dev_alloc<int32_t>(E, D.win_total);
   if (D.win_cols_kr) D.nd_cols_kr = dev_alloc<int32_t>(E, 3 * D.win_total);
-  hipLaunchKernelGGL(node_window_kernel, dim3((uint32_t)blocks), dim3(kNdWaves * 64), 0, stream,
+  hipLaunchKernelGGL(node_window_kernel, dim3((uint32_t)G), dim3(kNdWaves * 64), 0, stream,
                      D.win_idx, D.warp_offsets, D.max_nz_rows, D.win_off, D.win_cols,
-                     D.win_cols_kr, G, cnt, D.nd_off, D.nd_cols, D.nd_cols_kr, D.nd_pos);
+                     D.win_cols_kr, cnt, D.nd_off, D.nd_cols, D.nd_cols_kr, D.nd_pos);
   hip_check(hipGetLastError(), "node window launch");
   hip_check(hipStreamSynchronize(stream), "node windows");
   D.nd_cnt = cnt;
@@ -1723,11 +1724,9 @@ void build_packed_positions(wk_engine *E, DevLayout &D, hipStream_t stream) {
   }
   D.win_pk_off = dev_upload(E, off.data(), (int64_t)off.size(), stream);
   D.win_pk = dev_alloc<uint32_t>(E, (int64_t)off.back() * 64 * 4);
-  constexpr int wpb = 4;
-  const int64_t blocks = ((int64_t)D.ngroups + wpb - 1) / wpb;
   if (D.win_pk)
-    hipLaunchKernelGGL(pack_positions_kernel, dim3((uint32_t)blocks), dim3(wpb * 64), 0, stream,
-                       D.win_idx, D.warp_offsets, D.max_nz_rows, D.win_pk_off, D.ngroups,
+    hipLaunchKernelGGL(pack_positions_kernel, dim3((uint32_t)D.ngroups), dim3(256), 0, stream,
+                       D.win_idx, D.warp_offsets, D.max_nz_rows, D.win_pk_off,
                        reinterpret_cast<u32x4 *>(D.win_pk));
   hip_check(hipGetLastError(), "pack launch");
   hip_check(hipStreamSynchronize(stream), "pack");
