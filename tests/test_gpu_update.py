@@ -85,3 +85,18 @@ def test_update_values_row_sorted_and_device_scanned():
     assert np.array_equal(c.download(capi.WK_ENGINE_VALUES), s.process_host(new, m.colind)[0])
     for e in (a, b, c):
         e.close()
+
+
+@pytest.mark.parametrize("lens", [[1, 4, 3], [4], [5, 8, 1, 7], [8], [9, 7, 8]])
+@pytest.mark.parametrize("variant", [1, 2])
+def test_update_values_of_many_short_groups(lens, variant):
+    """4,097 groups of rows: the tiles of 4 and 8 steps (one wave a group), and past them."""
+    say(f"[gpu] update many {lens} {variant}")
+    m = matrix(64 * 4096 + 7, lens, seed=6)
+    s = scanned(m, variant, 64)
+    eng = engine(s, m.vals, m.colind)
+    new = np.random.default_rng(11).uniform(-1, 1, m.nnz)
+    eng.update_values(torch.from_numpy(new).cuda())
+    pv, _ = s.process_host(new, m.colind)
+    assert np.array_equal(eng.download(capi.WK_ENGINE_VALUES), pv)
+    eng.close()

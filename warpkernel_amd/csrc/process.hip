@@ -3,15 +3,15 @@
 // alone, on the device.
 //
 // Layouts whose lanes hold runs of CSR entries (every forward layout without
-// the row sort): one block per group reads its rows' entries 16 or 32 at a time,
+// the row sort): one block per group reads its rows' entries 4 to 64 at a time,
 // turns them around in LDS and writes whole steps.  It streams 16 bytes per
 // FP64 entry, both ways in whole lines, with no index array.  (One thread per
 // entry writing through the CSR-to-slot map put 8 bytes into each 128-byte
-// line: hex elasticity 48^3, 27.4M entries, 305 us against 83.)  The
+// line: hex elasticity 48^3, 27.4M entries, 305 us against 77.)  The
 // transposed layout reads the entry of each slot instead: indices and values
 // written in order, the 8-byte reads land on lines that the same group's other
 // steps read too (hex diffusion 48^3, both layouts 31 us as two scatters,
-// 24 here in one launch).
+// 23 here in one launch).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -23,7 +23,9 @@ namespace wk {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kGatherPer = 8;   // slots per thread of the transposed layout
+// slots per thread of the transposed layout (hex diffusion 48^3, the training
+// step: 54.9 us with 4, 57.0 with 8)
+constexpr int kGatherPer = 4;
 
 struct UpdateArgs {
   const void *src;                // CSR values
@@ -38,10 +40,11 @@ struct UpdateArgs {
   int32_t nblocks_t;              // blocks of the transposed layout
 };
 
-// S: steps of a group turned at a time
-template <class T, int W, int S>
+// S: steps of a group turned at a time, by TH threads
+template <class T, int W, int S, int TH>
 __device__ __forceinline__ void turn_group(const UpdateArgs &u, int32_t g) {
-  constexpr int PER = S * W / kThreads;
+  constexpr int PER = S * W / TH;
+  static_assert(PER * TH == S * W, "whole passes");
   __shared__ int2 ls[W];
   __shared__ T tile[W][S + 1];  // odd row length: the turned reads spread over the banks
   const int32_t tid = threadIdx.x;
@@ -54,31 +57,31 @@ __device__ __forceinline__ void turn_group(const UpdateArgs &u, int32_t g) {
     T v[PER];
 #pragma unroll
     for (int j = 0; j < PER; j++) {
-      const int2 s = ls[(tid + j * kThreads) / S];
-      const int32_t i = i0 + tid % S;
+      const int2 s = ls[(tid + j * TH) / S];
+      const int32_t i = i0 + (tid + j * TH) % S;
       v[j] = i < s.y ? src[s.x + i] : T(0);
     }
 #pragma unroll
-    for (int j = 0; j < PER; j++) tile[(tid + j * kThreads) / S][tid % S] = v[j];
+    for (int j = 0; j < PER; j++) tile[(tid + j * TH) / S][(tid + j * TH) % S] = v[j];
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < PER; j++) {
-      const int32_t l = tid % W, t = (tid + j * kThreads) / W;
+      const int32_t l = tid % W, t = (tid + j * TH) / W;
       if (i0 + t < len) dst[l + (int64_t)W * (i0 + t)] = tile[l][t];
     }
     __syncthreads();
   }
 }
 
-template <class T>
+template <class T, int TH>
 __device__ __forceinline__ void gather_slots(const UpdateArgs &u, int32_t b) {
   const T *src = static_cast<const T *>(u.src);
   T *dst = static_cast<T *>(u.dst_t);
-  const int64_t s0 = (int64_t)b * (kThreads * kGatherPer) + threadIdx.x;
+  const int64_t s0 = (int64_t)b * (TH * kGatherPer) + threadIdx.x;
   int32_t e[kGatherPer];
 #pragma unroll
   for (int j = 0; j < kGatherPer; j++) {
-    const int64_t s = s0 + (int64_t)j * kThreads;
+    const int64_t s = s0 + (int64_t)j * TH;
     e[j] = s < u.slots_t ? u.src_of_slot[s] : -1;
   }
   T v[kGatherPer];
@@ -86,18 +89,18 @@ __device__ __forceinline__ void gather_slots(const UpdateArgs &u, int32_t b) {
   for (int j = 0; j < kGatherPer; j++) v[j] = e[j] >= 0 ? src[e[j]] : T(0);
 #pragma unroll
   for (int j = 0; j < kGatherPer; j++)
-    if (e[j] >= 0) dst[s0 + (int64_t)j * kThreads] = v[j];
+    if (e[j] >= 0) dst[s0 + (int64_t)j * TH] = v[j];
 }
 
 // Blocks [0, ngroups): groups of the forward layout; then the transposed
 // layout's slots, each XCD a contiguous range of them.
-template <class T, int W, int S>
-__global__ __launch_bounds__(kThreads) void update_kernel(UpdateArgs u) {
+template <class T, int W, int S, int TH>
+__global__ __launch_bounds__(TH) void update_kernel(UpdateArgs u) {
   const int32_t b = blockIdx.x;
   if (b < u.ngroups)
-    turn_group<T, W, S>(u, b);
+    turn_group<T, W, S, TH>(u, b);
   else
-    gather_slots<T>(u, work_id(b - u.ngroups, u.nblocks_t, 1));
+    gather_slots<T, TH>(u, work_id(b - u.ngroups, u.nblocks_t, 1));
 }
 
 // Row-sorted layouts, whose lanes hold no runs: entry i to slot[i].
@@ -128,26 +131,41 @@ void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
                        static_cast<const T *>(vals), D.slot_of_nz, static_cast<T *>(D.vals), E->nnz);
     hip_check(hipGetLastError(), "scatter launch");
   }
+  // The steps turned at a time, by mean row length.  Up to 4 and 8, where there are
+  // groups enough, one wave a group: most of a 16-step tile and three of its waves
+  // would be empty (threshold 5, P1 tets 54^3, 10,399 groups, 14.1 -> 8.5 us, 9.6 by
+  // the map; threshold 4, 2D Laplacian 400^2 11.4 -> 6.4; with 2,246 groups level).
+  // Up to 16, half the LDS of 32 and twice the blocks in flight (2D Laplacian 407^2,
+  // 9 entries, residual with new values 15.1 -> 14.6); 32; and for longer rows 64 by eight waves, a whole
+  // group in two turns (hex elasticity, 81 entries: 48^3 residual with new values
+  // 129.1 -> 122.1 us, 123.2 with 32 steps and eight waves; 16^3 update 5.9 -> 5.1;
+  // but hex diffusion 60^3, 27 entries, 16.1 -> 17.4, and FP32 elasticity 28^3 8.4
+  // -> 9.0)
+  const int64_t slots = (int64_t)D.W * D.ngroups;
+  const bool many = D.ngroups >= 4096;
+  const int steps = D.W != 64                                       ? 32
+                    : many && D.allocate_nz <= 4 * slots            ? 4
+                    : many && D.allocate_nz <= 8 * slots            ? 8
+                    : D.allocate_nz <= 16 * slots                   ? 16
+                    : sizeof(T) == 4 || D.allocate_nz <= 32 * slots ? 32
+                                                                    : 64;
+  const int threads = steps <= 8 ? 64 : steps == 64 ? 512 : kThreads;
   if (E->has_adj) {
     u.dst_t = E->adj.vals;
     u.src_of_slot = E->adj.src_of_slot;
     u.slots_t = E->adj.allocate_nz;
-    u.nblocks_t = (int32_t)((u.slots_t + kThreads * kGatherPer - 1) / (kThreads * kGatherPer));
+    u.nblocks_t = (int32_t)((u.slots_t + threads * kGatherPer - 1) / (threads * kGatherPer));
   }
   const int64_t blocks = (int64_t)u.ngroups + u.nblocks_t;
   if (blocks > INT32_MAX) fail(WK_ERR_LIMIT, "grid too large");
   if (blocks == 0) return;
-  // 16 steps at a time where the rows are that short: half the LDS, twice the
-  // blocks in flight (2D Laplacian 407^2, 9 entries, residual with new values
-  // 15.1 -> 14.6 us)
-  const bool narrow = D.allocate_nz <= (int64_t)16 * D.W * D.ngroups;
-  const dim3 grid((uint32_t)blocks), block(kThreads);
-  if (D.W == 64 && narrow)
-    hipLaunchKernelGGL((update_kernel<T, 64, 16>), grid, block, 0, s, u);
-  else if (D.W == 64)
-    hipLaunchKernelGGL((update_kernel<T, 64, 32>), grid, block, 0, s, u);
-  else
-    hipLaunchKernelGGL((update_kernel<T, 32, 32>), grid, block, 0, s, u);
+  const auto kernel = D.W != 64     ? update_kernel<T, 32, 32, kThreads>
+                      : steps == 4  ? update_kernel<T, 64, 4, 64>
+                      : steps == 8  ? update_kernel<T, 64, 8, 64>
+                      : steps == 16 ? update_kernel<T, 64, 16, kThreads>
+                      : steps == 32 ? update_kernel<T, 64, 32, kThreads>
+                                    : update_kernel<T, 64, 64, 512>;
+  hipLaunchKernelGGL(kernel, dim3((uint32_t)blocks), dim3((uint32_t)threads), 0, s, u);
   hip_check(hipGetLastError(), "update launch");
 }
 
