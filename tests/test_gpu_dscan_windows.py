@@ -95,3 +95,23 @@ def test_windows_equal_the_host_built(name, variant):
     assert torch.equal(y0, y1)
     host.close()
     dev.close()
+
+
+def test_long_rows_are_scanned_when_the_call_returns():
+    """Rows past 128 entries have no windows: the engine built on one stream is
+    whole when the call returns, for any other stream."""
+    print("[gpu] device scan of long rows on a side stream", flush=True)
+    m = band(20000, [300, 150], 2000, 9)
+    host = engine(structure(64).scan(m.nnz, m.nrows, m.vals, m.rowptr, m.colind), m.vals, m.colind)
+    a = [torch.from_numpy(v).cuda() for v in (m.rowptr, m.colind, m.vals)]
+    x = torch.rand(m.ncols, dtype=torch.float64, device="cuda")
+    y0, y1 = (torch.full((m.nrows,), float("nan"), dtype=torch.float64, device="cuda") for _ in range(2))
+    host.launch(x, y0)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    dev = engine.from_device(*a, stream=side)
+    assert side.query()
+    dev.launch(x, y1)
+    assert torch.equal(y0, y1)
+    host.close()
+    dev.close()

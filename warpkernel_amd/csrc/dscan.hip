@@ -661,11 +661,14 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
     D.vals = dev_alloc<float>(E, D.allocate_nz);
     launch_fill<float>(D, rowptr, colind, vals, s);
   }
-  if (!G) hip_check(hipStreamSynchronize(s), "device scan");  // (else: the window counts' download)
 
   // 5. x windows, when every group fits
   const uint32_t longest = G ? *std::max_element(A.begin(), A.end()) : 0;
-  if (G && (int64_t)longest * 64 <= kWinSlots) {
+  const bool windows = G && (int64_t)longest * 64 <= kWinSlots;
+  // the uploads' host arrays go, and the caller may use the engine on another
+  // stream or free the CSR (with windows, their counts' download waits)
+  if (!windows) hip_check(hipStreamSynchronize(s), "device scan");
+  if (windows) {
     WinBuild wb{rowptr, D.row_map, D.row_map_inv, D.cols, D.warp_offsets, D.max_nz_rows,
                 D.tpr, D.row_off, nznrows};
     const int32_t stride = std::min((int32_t)longest * 64, kMaxWindow);
