@@ -168,3 +168,24 @@ def test_row_sets_default_and_column_swap():
     e32.launch(dev(xq), y)
     assert np.array_equal(y.cpu().numpy(), ref)  # FP64 sums by default here
     e32.close()
+
+
+@pytest.mark.parametrize("where", ["host", "device"])
+def test_row_sets_are_built_when_the_call_returns(where):
+    """An engine built on one stream is whole when the call returns, for any other."""
+    say(f"[gpu] row sets built on a side stream, {where}")
+    m = fe.hex_elastic_3d(24)
+    s = structure(64).scan(m.nnz, m.nrows, m.vals, m.rowptr, m.colind)
+    x = fe.uniform_x(m.ncols, 8, seed=6)
+    a = [dev(v) for v in (m.rowptr, m.colind, m.vals)]
+    dx, y = dev(x), out(m.nrows, 8)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    if where == "host":
+        eng = engine(s, m.vals, m.colind, stream=side)
+    else:
+        eng = engine.from_device(*a, stream=side)
+    assert side.query()
+    eng.launch(dx, y, cfg=SETS)
+    assert np.array_equal(y.cpu().numpy(), O.csr_spmv(m.rowptr, m.colind, m.vals, x))
+    eng.close()

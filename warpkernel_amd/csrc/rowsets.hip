@@ -409,7 +409,6 @@ void row_sets_finish(wk_engine *E, DevLayout &D, const uint64_t *starts, uint32_
   if (waves > INT32_MAX / 64 || (double)D.nznrows < kSetRows * (double)sets) return;
   D.rs_narrow = widest <= 65535;
   hip_check(hipMemcpyAsync(span, woff.data(), 4 * woff.size(), hipMemcpyHostToDevice, stream), "row sets");
-  hip_check(hipStreamSynchronize(stream), "row sets");
   // records, columns and Kr columns in one allocation
   const size_t n = (size_t)waves * kMaxChunks * 128;
   const size_t rec_bytes = sizeof(SetRec) * (size_t)waves, col_bytes = n * (D.rs_narrow ? 2 : 4);
@@ -431,6 +430,8 @@ void row_sets_finish(wk_engine *E, DevLayout &D, const uint64_t *starts, uint32_
                        D.max_nz_rows, starts, span, static_cast<int32_t *>(D.rs_cols_kr), nullptr);
     hip_check(hipGetLastError(), "row set launch");
   }
+  // woff goes, and the engine may be used on another stream
+  hip_check(hipStreamSynchronize(stream), "row sets");
   D.rs_waves = (int32_t)waves;
 }
 
