@@ -438,7 +438,8 @@ int wk_tune(wk_engine *engine, int32_t op, const wk_launch *base, const void *x_
 /* Read / replace the configuration the engine uses for (op, k) when cfg is
  * NULL (before tuning: a choice from the layout; FP32 engines get WK_ACC_F64
  * where the matrix cores sum, which is closer to the exact result than
- * WK_ACC_TWOSUM). */
+ * WK_ACC_TWOSUM; that configuration with WK_ACC_TWOSUM in its place runs as the
+ * windows' default for compensated sums). */
 int wk_engine_get_launch(const wk_engine *engine, int32_t op, int32_t k, wk_launch *cfg);
 int wk_engine_set_launch(wk_engine *engine, int32_t op, int32_t k, const wk_launch *cfg);
 

@@ -189,3 +189,24 @@ def test_row_sets_are_built_when_the_call_returns(where):
     eng.launch(dx, y, cfg=SETS)
     assert np.array_equal(y.cpu().numpy(), O.csr_spmv(m.rowptr, m.colind, m.vals, x))
     eng.close()
+
+
+@pytest.mark.parametrize("k", [5, 8, 9, 16])
+def test_compensated_sums_on_request(k):
+    """An FP32 engine asked for compensated sums on top of its default: the
+    windows' sums, bit for bit, each row's in the same order."""
+    say(f"[gpu] row sets, compensated sums k={k}")
+    m = fe.hex_elastic_3d(7)
+    s = structure(64).scan(m.nnz, m.nrows, m.vals, m.rowptr, m.colind)
+    eng = engine(s, m.vals, m.colind, dtype="f32")
+    assert eng.get_launch(k=k).accumulate == capi.WK_ACC_F64
+    x = dev(fe.uniform_x(m.ncols, k, seed=8).astype(np.float32))
+    y0, y1, y2, y3 = (out(m.nrows, k) for _ in range(4))
+    eng.launch(x, y0, cfg=dict(OTHER, accumulate=capi.WK_ACC_TWOSUM))
+    eng.launch(x, y1, cfg=dict(accumulate=capi.WK_ACC_TWOSUM))
+    eng.launch(x, y2)
+    eng.set_launch(dict(accumulate=capi.WK_ACC_TWOSUM), k=k)
+    eng.launch(x, y3)
+    a, b, c, d = (t.cpu().numpy() for t in (y0, y1, y2, y3))
+    assert np.array_equal(a, b) and np.array_equal(a, d) and not np.array_equal(a, c)
+    eng.close()

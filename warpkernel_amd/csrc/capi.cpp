@@ -249,7 +249,7 @@ void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double 
 }
 
 wk_launch resolve(wk_engine *E, int32_t op, int32_t k, const wk_launch *cfg) {
-  return cfg ? *cfg : engine_launch(E, op, k);
+  return compensated_launch(E, op, k, cfg ? *cfg : engine_launch(E, op, k));
 }
 
 void check_engine(const wk_engine *E) {

@@ -21,7 +21,9 @@
 // the matrix instructions alone take 18.  Measured and not kept: x through an
 // LDS window filled by direct-to-LDS loads (64^3 k=8 221 us, k=32 489), values
 // through LDS in 16-byte pieces (k=8 193), a ring of 3 or 21 steps (k=8 187,
-// 217), 20 waves per CU (spills: 307).
+// 217), 20 waves per CU (spills: 307), each lane's 32 bytes of a line of x as 16 of
+// each half (48^3 k=32 177 against 168), nontemporal values, whose lines the
+// neighbouring waves then miss (32^3 k=16 34.8 against 26.3).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

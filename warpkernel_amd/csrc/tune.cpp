@@ -133,7 +133,7 @@ std::vector<wk_launch> candidates(const DevLayout &D, int32_t dtype, const wk_la
 
 }  // namespace
 
-wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr) {
+wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr, bool f64_sums) {
   wk_launch c;
   wk_launch_default(&c);
   bool masked = false;  // k-tiles may exceed k (windowed multi-RHS)
@@ -369,7 +369,7 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
       }
     }
   }
-  if (D.rs_waves > 0 && win_ok && k >= 5 && (dtype == WK_F64 || k >= 9 || D.ngroups < 8192)) {
+  if (D.rs_waves > 0 && win_ok && k >= 5 && (dtype == WK_F64 || (f64_sums && (k >= 9 || D.ngroups < 8192)))) {
     // row sets on the matrix cores (stage 6, rowsets.hip), all of k in one
     // launch.  Hex elasticity, FP64: 32^3 k=5 18.1 us against 36.4, k=8 18.7
     // against 30.9, k=16 25.1 against 58.4, k=32 38.4 against 100; 64^3 k=5
@@ -399,7 +399,20 @@ wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k) {
     auto it = E->launch_cfg.find(cfg_key(op, k));
     if (it != E->launch_cfg.end()) return it->second;
   }
-  return heuristic_launch(layout_for(E, op), E->dtype, k, op == WK_OP_RUN_X);
+  return heuristic_launch(layout_for(E, op), E->dtype, k, op == WK_OP_RUN_X, true);
+}
+
+wk_launch compensated_launch(wk_engine *E, int32_t op, int32_t k, const wk_launch &c) {
+  if (E->dtype != WK_F32 || c.accumulate != WK_ACC_TWOSUM || c.stage_lds != 6) return c;
+  const DevLayout &D = layout_for(E, op);
+  const wk_launch d = heuristic_launch(D, E->dtype, k, op == WK_OP_RUN_X, true);
+  if (d.accumulate != WK_ACC_F64) return c;
+  wk_launch w = heuristic_launch(D, E->dtype, k, op == WK_OP_RUN_X, false);
+  for (int32_t wk_launch::*f : {&wk_launch::waves_per_block, &wk_launch::unroll, &wk_launch::k_tile,
+                                &wk_launch::xcd_remap, &wk_launch::nontemporal, &wk_launch::rows_per_lane,
+                                &wk_launch::blocks_per_cu})
+    if (c.*f != d.*f) w.*f = c.*f;
+  return w;
 }
 
 }  // namespace wk

@@ -280,7 +280,13 @@ int64_t dvals_tile_size();
 // The configuration an engine uses for (op, k) when the caller passes none:
 // the tuned one if any, else a choice from the layout.
 wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k);
-wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr);
+// f64_sums: FP32 engines may take the row sets, which sum in FP64.
+wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr, bool f64_sums);
+// The launch for c.  An FP32 engine whose default is the row sets has none of them
+// for compensated sums: where a caller overrides the default's accumulate alone or
+// with other fields, these go on top of the windows' default (hex elasticity 32^3
+// k=8 24.1 us against 31.3 with the default's stage 6, 48^3 k=32 256 against 357).
+wk_launch compensated_launch(wk_engine *E, int32_t op, int32_t k, const wk_launch &c);
 
 // WPK2's group split (warpkernel.hpp:633-691) over the longest row of each
 // W-row group of sorted rows (aw0); nzr = non-empty rows.  Outputs per
