@@ -254,7 +254,9 @@ def extra_multi_rhs(torch, dev, steps, warmup, tune=True, flusher=None):
         y32 = torch.empty((m.nrows, k), dtype=torch.float64, device="cuda")
         if tune:
             e64.tune(dx64, y64, reps=5)
-            e32.tune(dx32, y32, reps=5)
+            e32.tune(dx32, y32, reps=5, base=dict(accumulate=0))
+        else:
+            e32.set_launch(dict(accumulate=0), k=k)
         _, ms64 = time_launches(torch, lambda: e64.launch(dx64, y64), steps, warmup)
         _, ms32 = time_launches(torch, lambda: e32.launch(dx32, y32), steps, warmup)
         c64 = warm_cold(torch, lambda: e64.launch(dx64, y64), steps, flusher)
