@@ -377,7 +377,8 @@ int wk_run(wk_engine *engine, const wk_launch *cfg, const void *x_dev, double *y
 int wk_run_x(wk_engine *engine, const wk_launch *cfg, const void *x_dev, double *y_dev,
              int32_t k, int64_t ldx, int64_t ldy, void *stream);
 
-/* r = b - A x in FP64 (FP64 engines).  No reference counterpart. */
+/* r = b - A x in FP64 (FP64 engines); r may be b (same pointer, ldr = ldb).  No
+ * reference counterpart. */
 int wk_residual(wk_engine *engine, const wk_launch *cfg, const double *b_dev, int64_t ldb,
                 const double *x_dev, double *r_dev, int32_t k, int64_t ldx, int64_t ldr,
                 void *stream);

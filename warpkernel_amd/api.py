@@ -396,7 +396,7 @@ class engine:
         check(lib().wk_run_assembly(self._h, self._ref(c), _dev_ptr(y), _stream(stream)))
 
     def residual(self, b, x, r, cfg=None, stream=None):
-        """r = b - A x in FP64."""
+        """r = b - A x in FP64 (r may be b)."""
         k, ldx = self._k_ld(x)
         _, ldb = self._k_ld(b)
         _, ldr = self._k_ld(r)

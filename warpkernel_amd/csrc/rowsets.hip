@@ -110,8 +110,8 @@ __device__ __forceinline__ void rowset_wave(const SpmvArgs &a, const SetRec *rec
   const int32_t dst = OUT == OUT_RUNX ? rowid : a.row_map[rowid < a.nznrows ? rowid : a.nznrows - 1];
 
   // The lane's first column of tile t.  In a last tile of fewer than KT columns
-  // lanes move left onto columns that others hold too: the same sums, stored
-  // twice, and no masked reads (k >= E).
+  // lanes move left onto columns that others hold too: the same sums (y is
+  // stored twice), and no masked reads (k >= E).
   auto column = [&](int32_t t) {
     const int32_t c = t * KT + i4 * E;
     return c < a.k - E ? c : a.k - E;
@@ -134,12 +134,20 @@ __device__ __forceinline__ void rowset_wave(const SpmvArgs &a, const SetRec *rec
     if (!writer) return;
     const int32_t e0 = column(t);
     double *yr = a.y + (int64_t)dst * a.ldy + e0;
+    if constexpr (OUT == OUT_RESID) {
+      // r may be b: of a column that several lanes hold, only the one whose place
+      // it is in the tile may write, and all of b is read before
+      const double *br = a.b + (int64_t)dst * a.ldb + e0;
+      const int32_t others = t * KT + i4 * E - e0;  // leading columns of other lanes
+      double bv[E];
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-      if constexpr (OUT == OUT_RESID)
-        yr[e] = a.b[(int64_t)dst * a.ldb + e0 + e] - acc[e];
-      else
-        yr[e] = acc[e];
+      for (int e = 0; e < E; e++) bv[e] = br[e];
+#pragma unroll
+      for (int e = 0; e < E; e++)
+        if (e >= others) yr[e] = bv[e] - acc[e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; e++) yr[e] = acc[e];
     }
   };
   uint32_t tb = (uint32_t)column(0) * (uint32_t)sizeof(X);
