@@ -392,8 +392,10 @@ bool row_sets_begin(DevLayout &D, uint64_t *starts, uint32_t *span, hipStream_t 
   D.rs_waves = 0;
   const int32_t G = D.ngroups;
   if (D.variant != 1 || D.W != 64 || D.win_max <= 0 || G <= 0 || !D.cols) return false;
+  // (a group without steps, which only arrays from elsewhere can hold, has no last
+  // step to repeat)
   for (int32_t g = 0; g < G; g++)
-    if (set_chunks((int32_t)D.h_max_nz_rows[g]) > kMaxChunks) return false;
+    if (!D.h_max_nz_rows[g] || set_chunks((int32_t)D.h_max_nz_rows[g]) > kMaxChunks) return false;
   const int64_t blocks = ((int64_t)G + kBuildWaves - 1) / kBuildWaves;
   hipLaunchKernelGGL(row_set_kernel, dim3((uint32_t)blocks), dim3(kBuildWaves * 64), 0, stream, D.cols,
                      D.warp_offsets, D.max_nz_rows, G, starts, span);
