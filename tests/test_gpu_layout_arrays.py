@@ -77,3 +77,20 @@ def test_group_without_entries(k):
             assert np.all(np.abs(y.cpu().numpy() - ref) <= bound)
         eng.close()
     s.close()
+
+
+def test_groups_without_rows():
+    """Split groups, none of whose rows counts as one with entries: y is 0."""
+    say("[gpu] layout without rows that count")
+    n, lens = 130, [2, 1]
+    rp = np.minimum(np.arange(n + 1), 60).astype(np.int32)  # 60 rows of one entry
+    s = layout(2, n, 0, rp, np.arange(n), np.arange(60), lens, tpr=[1, 1], row_off=[0, 64, n])
+    colind = np.arange(60, dtype=np.int32)
+    eng = engine(s, np.full(60, 2.0), colind)
+    x = torch.ones(n, dtype=torch.float64, device="cuda")
+    for cfg in (None, dict(stage_lds=0, unroll=8, nontemporal=1, rows_per_lane=1, k_tile=1)):
+        y = torch.full((n,), float("nan"), dtype=torch.float64, device="cuda")
+        eng.launch(x, y, cfg=cfg)
+        assert torch.equal(y, torch.zeros_like(y)), cfg
+    eng.close()
+    s.close()

@@ -174,8 +174,9 @@ bool deltas_begin(wk_engine *E, DevLayout &D, std::vector<uint32_t> &off, uint32
                   hipStream_t stream) {
   const int32_t G = D.ngroups;
   // short rows whose windows do not pay by themselves (swapped columns turn
-  // the windows off, and the offsets with them)
-  if (D.W != 64 || D.win_max <= 0 || D.nd_max > 0 || G <= 0 ||
+  // the windows off, and the offsets with them); lanes past the last row with
+  // entries read its place in row_map, so there has to be one
+  if (D.W != 64 || D.nznrows <= 0 || D.win_max <= 0 || D.nd_max > 0 || G <= 0 ||
       (double)D.allocate_nz >= 40.0 * 64.0 * (double)G || (double)D.allocate_nz < 1.25 * (double)D.win_total)
     return false;
   off.assign((size_t)G + 1, 0);
