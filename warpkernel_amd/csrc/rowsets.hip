@@ -222,14 +222,16 @@ __global__ __launch_bounds__(kSetBlock * 64, (set_waves<P, E>())) void spmv_rows
 }
 
 // Row sets of one group per wave: lanes in order, a lane joins the set of the
-// lane before it when both read the same column at every step and the set has
-// fewer than four lanes.  Pass 1 writes a bit per lane that starts a set and
-// the widest column span of a lane.
+// lane before it when both read the same column at every step, in Kr numbering
+// too, and the set has fewer than four lanes.  (A pad and an entry of column 0
+// read the same column of x but not of x in Kr numbering, where pads read column
+// 0 too.)  Pass 1 writes a bit per lane that starts a set and the widest column
+// span of a lane.
 constexpr int kBuildWaves = 4;
 __global__ __launch_bounds__(kBuildWaves * 64) void row_set_kernel(
-    const int32_t *__restrict__ cols, const int64_t *__restrict__ warp_offsets,
-    const uint32_t *__restrict__ max_nz_rows, int32_t ngroups, uint64_t *__restrict__ starts,
-    uint32_t *__restrict__ span) {
+    const int32_t *__restrict__ cols, const int32_t *__restrict__ cols_kr,
+    const int64_t *__restrict__ warp_offsets, const uint32_t *__restrict__ max_nz_rows, int32_t ngroups,
+    uint64_t *__restrict__ starts, uint32_t *__restrict__ span) {
   const int32_t lane = threadIdx.x & 63;
   const int32_t g = __builtin_amdgcn_readfirstlane((int32_t)(blockIdx.x * kBuildWaves + (threadIdx.x >> 6)));
   if (g >= ngroups) return;
@@ -246,6 +248,10 @@ __global__ __launch_bounds__(kBuildWaves * 64) void row_set_kernel(
     for (int u = 0; u < U; u++) {
       const int32_t before = __shfl_up(p[u], 1);  // by every lane, also those that differ already
       same = same && before == p[u];
+      if (cols_kr && __ballot(p[u] == 0)) {
+        const int32_t kr = cols_kr[base + lane + 64 * (int64_t)(t0 + u < len ? t0 + u : len - 1)];
+        same = __shfl_up(kr, 1) == kr && same;
+      }
       lo = min(lo, p[u]);
       hi = max(hi, p[u]);
     }
@@ -398,7 +404,7 @@ bool row_sets_begin(DevLayout &D, uint64_t *starts, uint32_t *span, hipStream_t 
     if (!D.h_max_nz_rows[g] || set_chunks((int32_t)D.h_max_nz_rows[g]) > kMaxChunks) return false;
   const int64_t blocks = ((int64_t)G + kBuildWaves - 1) / kBuildWaves;
   hipLaunchKernelGGL(row_set_kernel, dim3((uint32_t)blocks), dim3(kBuildWaves * 64), 0, stream, D.cols,
-                     D.warp_offsets, D.max_nz_rows, G, starts, span);
+                     D.cols_kr, D.warp_offsets, D.max_nz_rows, G, starts, span);
   hip_check(hipGetLastError(), "row set launch");
   return true;
 }
