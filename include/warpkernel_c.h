@@ -346,21 +346,40 @@ typedef struct wk_launch {
                               right-hand sides through a window of that
                               many values per column; the rest of k (fewer
                               than one tile), and engines it does not fit,
-                              run as 4; where neighbouring rows share their
-                              columns (block matrices, WPK1, at most 84
-                              steps) FP64 engines, and FP32 ones with
-                              WK_ACC_F64, run all of k on the matrix cores
-                              instead, each row's sum in the same order; 7 (k_tile 1, engines with node
+                              run as 4; from five right-hand sides where
+                              neighbouring rows share their columns (block
+                              matrices, WPK1, at most 84 steps) FP64
+                              engines, and FP32 ones with WK_ACC_F64, run
+                              all of k on the matrix cores instead, each
+                              row's sum in the same order; 7 (k_tile 1, engines with node
                               windows; run, run_x and the residual): as 5, with a
                               window of node entries (three x values at
                               columns 3n .. 3n+2, or one column thrice for
                               pads; run_x: three Kr columns each) and one
                               10-bit entry index per three steps (unroll
                               16: 27-step batches, 8: 18-step); otherwise
-                              as 5 */
+                              as 5; 0 (direct loads) reads 16-bit column
+                              offsets instead of the columns where the
+                              layout has them (banded short rows; k_tile 1,
+                              unroll 8 or 16, nontemporal 1); 8: as 6,
+                              never on the matrix cores; 9: as 0, always
+                              the columns */
 } wk_launch;
 
 void wk_launch_default(wk_launch *cfg);
+
+/* The kinds of kernel the calling thread's last product (wk_run, wk_run_x,
+ * wk_residual, wk_run_adjoint) launched, a bit each; a shape that a layout does
+ * not offer runs as another. */
+#define WK_KERNEL_DIRECT 1      /* stage_lds 0 and 9 */
+#define WK_KERNEL_STAGED 2      /* 1, 2 */
+#define WK_KERNEL_WINDOWS 4     /* 3, 4 */
+#define WK_KERNEL_PACKED 8      /* 5 */
+#define WK_KERNEL_REGISTERS 16  /* 6 and 8: the window kernel with the values in registers */
+#define WK_KERNEL_ROW_SETS 32   /* 6: the matrix cores */
+#define WK_KERNEL_NODES 64      /* 7 */
+#define WK_KERNEL_OFFSETS 128   /* 0: 16-bit column offsets */
+uint32_t wk_last_kernels(void);
 
 /* engine::run (warpkernel.hpp:811-860): y[row_map[i]] = sum over group slots.
  * Asynchronous on `stream`.  Rows without nonzeros are written as 0 (the
@@ -439,9 +458,12 @@ int wk_tune(wk_engine *engine, int32_t op, const wk_launch *base, const void *x_
 /* Read / replace the configuration the engine uses for (op, k) when cfg is
  * NULL (before tuning: a choice from the layout; FP32 engines get WK_ACC_F64
  * where the matrix cores sum, which is closer to the exact result than
- * WK_ACC_TWOSUM; that configuration with WK_ACC_TWOSUM in its place runs as the
- * windows' default for compensated sums). */
+ * WK_ACC_TWOSUM).  wk_engine_get_launch_sums: the one it would use for sums of the
+ * given kind (WK_ACC_*; FP64 engines: the same), to pass or set where other sums
+ * are wanted than the engine's choice. */
 int wk_engine_get_launch(const wk_engine *engine, int32_t op, int32_t k, wk_launch *cfg);
+int wk_engine_get_launch_sums(const wk_engine *engine, int32_t op, int32_t k, int32_t accumulate,
+                              wk_launch *cfg);
 int wk_engine_set_launch(wk_engine *engine, int32_t op, int32_t k, const wk_launch *cfg);
 
 /* ------------------------------------------------------ batches and graphs */

@@ -106,6 +106,8 @@ SIGNATURES = {
     "wk_tune": (C.c_int, [P, I32, C.POINTER(Launch), P, P, I32, I64, I64, I32, P, C.POINTER(Launch),
                           C.POINTER(C.c_float)]),
     "wk_engine_get_launch": (C.c_int, [P, I32, I32, C.POINTER(Launch)]),
+    "wk_engine_get_launch_sums": (C.c_int, [P, I32, I32, I32, C.POINTER(Launch)]),
+    "wk_last_kernels": (U32, []),
     "wk_engine_set_launch": (C.c_int, [P, I32, I32, C.POINTER(Launch)]),
     "wk_batch_create": (C.c_int, [C.POINTER(C.c_void_p), I32, I32, I32, PP]),
     "wk_batch_bind": (C.c_int, [P, C.POINTER(C.c_void_p), C.POINTER(C.c_void_p), I32,
@@ -118,6 +120,8 @@ SIGNATURES = {
     "wk_graph_destroy": (None, [P]),
 }
 WK_OP_RUN, WK_OP_RUN_X, WK_OP_ADJOINT = 0, 1, 2
+WK_KERNEL_DIRECT, WK_KERNEL_STAGED, WK_KERNEL_WINDOWS, WK_KERNEL_PACKED = 1, 2, 4, 8
+WK_KERNEL_REGISTERS, WK_KERNEL_ROW_SETS, WK_KERNEL_NODES, WK_KERNEL_OFFSETS = 16, 32, 64, 128
 
 _lib = None
 

@@ -311,12 +311,17 @@ class engine:
         check(lib().wk_engine_set_launch(self._h, op, k, C.byref(c)))
 
     def _cfg(self, op, k, cfg):
-        """None -> NULL (engine's own choice); dict -> overrides on top of it."""
+        """None -> NULL (engine's own choice); dict -> overrides on top of it, or, where
+        it names the sums (accumulate), on top of the engine's choice for those."""
         if cfg is None:
             return None
         if isinstance(cfg, capi.Launch):
             return cfg
-        c = self.get_launch(op, k)
+        if "accumulate" in cfg:
+            c = capi.Launch()
+            check(lib().wk_engine_get_launch_sums(self._h, op, k, int(cfg["accumulate"]), C.byref(c)))
+        else:
+            c = self.get_launch(op, k)
         for key, v in cfg.items():
             if not hasattr(c, key):
                 raise KeyError(key)

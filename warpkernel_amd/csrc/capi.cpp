@@ -18,6 +18,8 @@ namespace {
 thread_local std::string g_last_error;
 }
 
+thread_local uint32_t g_launched = 0;
+
 void set_last_error(const std::string &msg) { g_last_error = msg; }
 
 [[noreturn]] void fail(int code, const std::string &msg) { throw Error{code, msg}; }
@@ -249,7 +251,7 @@ void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double 
 }
 
 wk_launch resolve(wk_engine *E, int32_t op, int32_t k, const wk_launch *cfg) {
-  return compensated_launch(E, op, k, cfg ? *cfg : engine_launch(E, op, k));
+  return cfg ? *cfg : engine_launch(E, op, k);
 }
 
 void check_engine(const wk_engine *E) {
@@ -593,6 +595,8 @@ int wk_engine_get_colinds(const wk_engine *E, int32_t *pcols_host) {
     hip_check(hipMemcpy(pcols_host, E->fwd.cols, bytes, hipMemcpyDeviceToHost), "get_colinds");
   });
 }
+
+uint32_t wk_last_kernels(void) { return g_launched; }
 
 void wk_launch_default(wk_launch *cfg) {
   if (!cfg) return;

@@ -1196,11 +1196,17 @@ int ceil_pow2(int v) {
 
 }  // namespace
 
-void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int out, const void *x,
+void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &launch, int out, const void *x,
                  int64_t ldx, double *y, int64_t ldy, const double *b, int64_t ldb, int32_t k,
                  hipStream_t stream) {
   if (k < 1) fail(WK_ERR_ARG, "k must be >= 1");
-  if (cfg.stage_lds < 0 || cfg.stage_lds > 7) fail(WK_ERR_ARG, "stage_lds must be 0 to 7");
+  if (launch.stage_lds < 0 || launch.stage_lds > 9) fail(WK_ERR_ARG, "stage_lds must be 0 to 9");
+  // 8 and 9: 6 and 0 without the row sets and the column offsets
+  wk_launch cfg = launch;
+  const bool compact = cfg.stage_lds < 8;
+  if (!compact) cfg.stage_lds = cfg.stage_lds == 8 ? 6 : 0;
+  uint32_t &launched = g_launched;
+  launched = 0;
   if (cfg.nontemporal < 0 || cfg.nontemporal > 2) fail(WK_ERR_ARG, "nontemporal must be 0, 1 or 2");
   const int wpb = cfg.waves_per_block;
   if (wpb != 1 && wpb != 2 && wpb != 4 && wpb != 8) fail(WK_ERR_ARG, "waves_per_block must be 1, 2, 4 or 8");
@@ -1235,13 +1241,16 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
   }
 
   int32_t j0 = 0;
-  // stage 6 on layouts with row sets (FP64, or FP32 values with FP64 sums): the
-  // matrix cores, all of k in one launch
-  if (cfg.stage_lds == 6 && rpl == 1 && cfg.nontemporal) {
+  // stage 6 on layouts with row sets (FP64, or FP32 values with FP64 sums) from
+  // kRowSetColumns: the matrix cores, all of k in one launch
+  if (cfg.stage_lds == 6 && compact && rpl == 1 && cfg.nontemporal) {
     a.x = x;
     a.y = y;
     a.b = b;
-    if (launch_rowsets(D, prec, out, a, k, cfg.xcd_remap ? 1 : 0, stream)) return;
+    if (launch_rowsets(D, prec, out, a, k, cfg.xcd_remap ? 1 : 0, stream)) {
+      launched = WK_KERNEL_ROW_SETS;
+      return;
+    }
   }
   // stage 6: the group's values in registers, one pass per 32-byte k-tile
   // (4 FP64 or 8 FP32 right-hand sides), all passes of a group in one wave;
@@ -1271,6 +1280,7 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
         rf(a, w, dim3((uint32_t)(nwork + nf)), dim3(wpb * 64), std::max(win_bytes * (size_t)wpb, lds),
            (int32_t)nwork, ntiles, cfg.xcd_remap ? 1 : 0, stream);
       hip_check(hipGetLastError(), "spmv launch");
+      launched |= WK_KERNEL_REGISTERS;
       j0 = ntiles * ktr;
     }
   }
@@ -1347,6 +1357,7 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
                (int32_t)nwork, cfg.xcd_remap ? 1 : 0, stream);
           hip_check(hipGetLastError(), "spmv launch");
         }
+        launched |= WK_KERNEL_NODES;
         j0 += ntiles;
         continue;
       }
@@ -1381,6 +1392,7 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
                cfg.xcd_remap ? 1 : 0, stream);
           hip_check(hipGetLastError(), "spmv launch");
         }
+        launched |= WK_KERNEL_PACKED;
         j0 += ntiles;
         continue;
       }
@@ -1424,6 +1436,7 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
           wf(a, w, dim3((uint32_t)(nwork + nf)), dim3(bw * 64), std::max(need, lds), (int32_t)nwork,
              ntiles, cfg.xcd_remap ? 1 : 0, stream);
         hip_check(hipGetLastError(), "spmv launch");
+        launched |= WK_KERNEL_WINDOWS;
         j0 += a.k;
         continue;
       }
@@ -1452,17 +1465,19 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
              cfg.xcd_remap ? 1 : 0, stream);
         hip_check(hipGetLastError(), "spmv launch");
       }
+      launched |= WK_KERNEL_STAGED;
       j0 += ntiles;
       continue;
     }
     // 16-bit column offsets in place of the direct kernel's columns
-    if (kt == 1 && ntiles == 1 && r == 1 && cfg.stage_lds == 0 && cfg.nontemporal == 1 && lds == 0 &&
+    if (kt == 1 && ntiles == 1 && r == 1 && cfg.stage_lds == 0 && compact && cfg.nontemporal == 1 && lds == 0 &&
         (cfg.unroll == 8 || cfg.unroll == 16)) {
       a.x = static_cast<const char *>(x) + (size_t)j0 * xsz;
       a.y = y + j0;
       a.b = b ? b + j0 : nullptr;
       a.k = 1;
       if (launch_deltas(D, prec, out, a, wpb, cfg.unroll, cfg.xcd_remap ? 1 : 0, stream)) {
+        launched |= WK_KERNEL_OFFSETS;
         j0 += 1;
         continue;
       }
@@ -1483,6 +1498,7 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
       fn(a, dim3((uint32_t)(nwork + nfill)), dim3(wpb * 64), lds, (int32_t)nwork, ntiles,
          cfg.xcd_remap ? 1 : 0, stream);
     hip_check(hipGetLastError(), "spmv launch");
+    launched |= WK_KERNEL_DIRECT;
     j0 += ntiles * kt;
   }
 }

@@ -33,6 +33,11 @@ int pow2_at_least(int v) {
 
 const DevLayout &layout_for(const wk_engine *E, int32_t op) { return op == WK_OP_ADJOINT ? E->adj : E->fwd; }
 
+// Whether stage 6 is the row sets.
+bool row_sets_run(const DevLayout &D, int32_t dtype, int32_t k, int32_t sums) {
+  return D.rs_waves > 0 && D.win_max > 0 && k >= kRowSetColumns && (dtype == WK_F64 || sums == WK_ACC_F64);
+}
+
 // Candidate set: the knobs that change speed but not results.
 std::vector<wk_launch> candidates(const DevLayout &D, int32_t dtype, const wk_launch &base, int32_t k) {
   std::vector<wk_launch> out;
@@ -50,6 +55,12 @@ std::vector<wk_launch> candidates(const DevLayout &D, int32_t dtype, const wk_la
           c.rows_per_lane = 1;
           c.stage_lds = 0;
           out.push_back(c);
+          if (D.dl_words) {
+            // the columns themselves where 0 takes their offsets
+            c.stage_lds = 9;
+            out.push_back(c);
+            c.stage_lds = 0;
+          }
           if (u == 8 && D.W == 64) {
             // the index stream nontemporal too (scattered x gathers keep more L2)
             c.nontemporal = 2;
@@ -118,10 +129,18 @@ std::vector<wk_launch> candidates(const DevLayout &D, int32_t dtype, const wk_la
             c.stage_lds = 0;
           }
         }
-        // the group's values held in registers across 32-byte k-tiles (the
-        // launcher falls back where groups are longer than 84 steps)
-        if (D.win_pk && k >= (int)(32 / vsz) && wpb <= 4) {
+        // the row sets (one shape), and the group's values held in registers
+        // across 32-byte k-tiles (the launcher falls back where groups are
+        // longer than 84 steps)
+        const bool sets = row_sets_run(D, dtype, k, base.accumulate);
+        if (sets && wpb == 1) {
           c.stage_lds = 6;
+          c.k_tile = std::min(8, pow2_at_most(k));
+          out.push_back(c);
+          c.stage_lds = 0;
+        }
+        if (D.win_pk && k >= (int)(32 / vsz) && wpb <= 4) {
+          c.stage_lds = sets ? 8 : 6;
           c.k_tile = std::min(32, pow2_at_most(k));
           out.push_back(c);
           c.stage_lds = 0;
@@ -133,7 +152,7 @@ std::vector<wk_launch> candidates(const DevLayout &D, int32_t dtype, const wk_la
 
 }  // namespace
 
-wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr, bool f64_sums) {
+wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr, int32_t sums) {
   wk_launch c;
   wk_launch_default(&c);
   bool masked = false;  // k-tiles may exceed k (windowed multi-RHS)
@@ -369,7 +388,9 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
       }
     }
   }
-  if (D.rs_waves > 0 && win_ok && k >= 5 && (dtype == WK_F64 || (f64_sums && (k >= 9 || D.ngroups < 8192)))) {
+  if (dtype != WK_F64 && sums != kDefaultSums) c.accumulate = sums;
+  if (win_ok && row_sets_run(D, dtype, k, sums == kDefaultSums ? WK_ACC_F64 : sums) &&
+      (dtype == WK_F64 || k >= 9 || D.ngroups < 8192)) {
     // row sets on the matrix cores (stage 6, rowsets.hip), all of k in one
     // launch.  Hex elasticity, FP64: 32^3 k=5 18.1 us against 36.4, k=8 18.7
     // against 30.9, k=16 25.1 against 58.4, k=32 38.4 against 100; 64^3 k=5
@@ -393,26 +414,21 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
   return c;
 }
 
-wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k) {
+wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k, int32_t sums) {
+  const DevLayout &D = layout_for(E, op);
   {
     std::lock_guard<std::mutex> g(E->cfg_mu);
     auto it = E->launch_cfg.find(cfg_key(op, k));
-    if (it != E->launch_cfg.end()) return it->second;
+    if (it != E->launch_cfg.end()) {
+      wk_launch c = it->second;
+      if (E->dtype == WK_F64 || sums == kDefaultSums || sums == c.accumulate) return c;
+      if (sums == WK_ACC_F64 || c.stage_lds != 6 || !row_sets_run(D, E->dtype, k, WK_ACC_F64)) {
+        c.accumulate = sums;
+        return c;
+      }
+    }
   }
-  return heuristic_launch(layout_for(E, op), E->dtype, k, op == WK_OP_RUN_X, true);
-}
-
-wk_launch compensated_launch(wk_engine *E, int32_t op, int32_t k, const wk_launch &c) {
-  if (E->dtype != WK_F32 || c.accumulate != WK_ACC_TWOSUM || c.stage_lds != 6) return c;
-  const DevLayout &D = layout_for(E, op);
-  const wk_launch d = heuristic_launch(D, E->dtype, k, op == WK_OP_RUN_X, true);
-  if (d.accumulate != WK_ACC_F64) return c;
-  wk_launch w = heuristic_launch(D, E->dtype, k, op == WK_OP_RUN_X, false);
-  for (int32_t wk_launch::*f : {&wk_launch::waves_per_block, &wk_launch::unroll, &wk_launch::k_tile,
-                                &wk_launch::xcd_remap, &wk_launch::nontemporal, &wk_launch::rows_per_lane,
-                                &wk_launch::blocks_per_cu})
-    if (c.*f != d.*f) w.*f = c.*f;
-  return w;
+  return heuristic_launch(D, E->dtype, k, op == WK_OP_RUN_X, sums);
 }
 
 }  // namespace wk
@@ -427,6 +443,15 @@ int wk_engine_get_launch(const wk_engine *E, int32_t op, int32_t k, wk_launch *c
     return WK_ERR_ARG;
   }
   *cfg = engine_launch(const_cast<wk_engine *>(E), op, k);
+  return WK_OK;
+}
+
+int wk_engine_get_launch_sums(const wk_engine *E, int32_t op, int32_t k, int32_t accumulate, wk_launch *cfg) {
+  if (!E || !cfg || op < 0 || op > 2 || k < 1) {
+    set_last_error("bad argument");
+    return WK_ERR_ARG;
+  }
+  *cfg = engine_launch(const_cast<wk_engine *>(E), op, k, accumulate == WK_ACC_F64 ? WK_ACC_F64 : WK_ACC_TWOSUM);
   return WK_OK;
 }
 

@@ -207,6 +207,8 @@ enum Out { OUT_RUN = 0, OUT_RUNX = 1, OUT_RESID = 2 };
 
 // Launches one SpMV over a device layout.  prec: WK_F64, or WK_F32 with
 // cfg.accumulate.  Throws wk::Error on unsupported options.
+// WK_KERNEL_* of the calling thread's last launch_spmv.
+extern thread_local uint32_t g_launched;
 void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int out,
                  const void *x, int64_t ldx, double *y, int64_t ldy, const double *b,
                  int64_t ldb, int32_t k, hipStream_t stream);
@@ -240,6 +242,9 @@ void row_sets_finish(wk_engine *E, DevLayout &D, const uint64_t *starts, uint32_
 bool deltas_begin(wk_engine *E, DevLayout &D, std::vector<uint32_t> &off, uint32_t *fits, uint32_t *dev_off,
                   hipStream_t stream);
 void deltas_finish(DevLayout &D, const uint32_t *fits);
+// Right-hand sides from which the row sets run: below, the windows read less (hex
+// elasticity 64^3 k=4 118 us against 175; 32^3 17.5 either way).
+constexpr int32_t kRowSetColumns = 5;
 // k right-hand sides through the row sets.  prec: 0 FP64, 2 FP32 values with
 // FP64 accumulation.  Returns false, nothing launched, where the layout or the
 // vectors do not allow it.
@@ -279,14 +284,13 @@ int64_t dvals_tile_size();
 
 // The configuration an engine uses for (op, k) when the caller passes none:
 // the tuned one if any, else a choice from the layout.
-wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k);
-// f64_sums: FP32 engines may take the row sets, which sum in FP64.
-wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr, bool f64_sums);
-// The launch for c.  An FP32 engine whose default is the row sets has none of them
-// for compensated sums: where a caller overrides the default's accumulate alone or
-// with other fields, these go on top of the windows' default (hex elasticity 32^3
-// k=8 24.1 us against 31.3 with the default's stage 6, 48^3 k=32 256 against 357).
-wk_launch compensated_launch(wk_engine *E, int32_t op, int32_t k, const wk_launch &c);
+// sums: WK_ACC_* for FP32 engines, kDefaultSums for the engine's choice (a tuned
+// configuration is the row sets' only where they may sum as asked, else the
+// layout's choice for those sums: hex elasticity 32^3 k=8 compensated 24.1 us
+// against 31.3 with the row sets' other fields, 48^3 k=32 256 against 357).
+constexpr int32_t kDefaultSums = -1;
+wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k, int32_t sums = kDefaultSums);
+wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr, int32_t sums);
 
 // WPK2's group split (warpkernel.hpp:633-691) over the longest row of each
 // W-row group of sorted rows (aw0); nzr = non-empty rows.  Outputs per
