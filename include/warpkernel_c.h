@@ -457,8 +457,9 @@ int wk_tune(wk_engine *engine, int32_t op, const wk_launch *base, const void *x_
 
 /* Read / replace the configuration the engine uses for (op, k) when cfg is
  * NULL (before tuning: a choice from the layout; FP32 engines get WK_ACC_F64
- * where the matrix cores sum, which is closer to the exact result than
- * WK_ACC_TWOSUM).  wk_engine_get_launch_sums: the one it would use for sums of the
+ * from five right-hand sides on where neighbouring rows share their columns
+ * (the layouts of the matrix cores' kernel, whatever their size), which is
+ * closer to the exact result than WK_ACC_TWOSUM).  wk_engine_get_launch_sums: the one it would use for sums of the
  * given kind (WK_ACC_*; FP64 engines: the same), to pass or set where other sums
  * are wanted than the engine's choice. */
 int wk_engine_get_launch(const wk_engine *engine, int32_t op, int32_t k, wk_launch *cfg);

@@ -144,3 +144,30 @@ def test_stage_0_and_9():
             eng.launch(dev(x), y, cfg=dict(BASE, k_tile=1, stage_lds=stage))
         assert e.value.code == capi.WK_ERR_ARG
     eng.close()
+
+
+@pytest.mark.parametrize("nodes", [60, 175000])
+def test_fp32_default_sums_do_not_depend_on_the_size(nodes):
+    """8,204 groups as one: FP64 sums from five right-hand sides where rows share
+    their columns, compensated ones below."""
+    say(f"[gpu] FP32 default sums, {nodes} nodes")
+    n = 3 * nodes
+    node = np.arange(nodes)
+    nb = np.sort(np.stack([node, (node + 1) % nodes], 1), 1)
+    ci = np.repeat((nb[:, :, None] * 3 + np.arange(3)).reshape(nodes, 6), 3, 0).reshape(-1).astype(np.int32)
+    m = fe.CSR("pairs", n, n, (6 * np.arange(n + 1)).astype(np.int32), ci,
+               np.random.default_rng(1).uniform(-1, 1, ci.size))
+    eng = engine(scan(m), m.vals, m.colind, dtype="f32")
+    v = m.vals.astype(np.float32).astype(np.float64)
+    for k in (4, 5, 8, 9):
+        assert eng.get_launch(k=k).accumulate == (capi.WK_ACC_F64 if k >= 5 else capi.WK_ACC_TWOSUM), k
+        xq = fe.uniform_x(n, k, seed=9).astype(np.float32)
+        y = out(n, k)
+        eng.launch(dev(xq), y)
+        if k >= 5:
+            assert np.array_equal(y.cpu().numpy(), O.csr_spmv(m.rowptr, ci, v, xq.astype(np.float64))), k
+        eng.launch(dev(xq), y, cfg=dict(accumulate=capi.WK_ACC_TWOSUM))
+        other = out(n, k)
+        eng.launch(dev(xq), other, cfg=dict(BASE, stage_lds=4, accumulate=capi.WK_ACC_TWOSUM))
+        assert torch.equal(y, other), k
+    eng.close()

@@ -38,6 +38,16 @@ bool row_sets_run(const DevLayout &D, int32_t dtype, int32_t k, int32_t sums) {
   return D.rs_waves > 0 && D.win_max > 0 && k >= kRowSetColumns && (dtype == WK_F64 || sums == WK_ACC_F64);
 }
 
+// The sums of an FP32 engine that is not told: FP64 ones from kRowSetColumns where
+// the layout has row sets, whichever kernel runs, so that they depend on k and the
+// matrix's structure and not on its size (they did: compensated up to k = 8 from
+// 8,192 groups, where 64^3 k=5 took 186 us against 122 here).  Exact products:
+// closer to the exact result than the compensated sums (1e-16 against 2e-14
+// normwise on 32^3), and faster (32^3 k=8 13.7 us against 23.5).
+int32_t default_sums(const DevLayout &D, int32_t k) {
+  return D.rs_waves > 0 && k >= kRowSetColumns ? WK_ACC_F64 : WK_ACC_TWOSUM;
+}
+
 // Candidate set: the knobs that change speed but not results.
 std::vector<wk_launch> candidates(const DevLayout &D, int32_t dtype, const wk_launch &base, int32_t k) {
   std::vector<wk_launch> out;
@@ -388,26 +398,21 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
       }
     }
   }
-  if (dtype != WK_F64 && sums != kDefaultSums) c.accumulate = sums;
-  if (win_ok && row_sets_run(D, dtype, k, sums == kDefaultSums ? WK_ACC_F64 : sums) &&
-      (dtype == WK_F64 || k >= 9 || D.ngroups < 8192)) {
+  if (dtype != WK_F64) c.accumulate = sums != kDefaultSums ? sums : default_sums(D, k);
+  if (win_ok && row_sets_run(D, dtype, k, c.accumulate) && (dtype == WK_F64 || k >= 9 || D.ngroups < 8192)) {
     // row sets on the matrix cores (stage 6, rowsets.hip), all of k in one
     // launch.  Hex elasticity, FP64: 32^3 k=5 18.1 us against 36.4, k=8 18.7
     // against 30.9, k=16 25.1 against 58.4, k=32 38.4 against 100; 64^3 k=5
     // 176 against 194, k=8 181 against 204, k=16 248 against 421, k=32 382
-    // against 803.  Up to k = 4 the windows read less: 32^3 k=4 17.5 either
-    // way, 64^3 175 against 118.  FP32 values: FP64 sums, exact products, so
-    // the result is closer to the exact one than the compensated FP32 sums'
-    // (1e-16 against 2e-14 normwise on 32^3) at 13.7 us against 23.5 (32^3
-    // k=8; 36.4 against 69 on 48^3); the 64^3 layout (12,874 groups) keeps
-    // its windows up to k = 8.
+    // against 803.  FP32 values with FP64 sums: 32^3 k=8 13.7 us, 48^3 36.4;
+    // large layouts keep their windows up to k = 8 (64^3, 12,874 groups, k=8
+    // 114 us against 126; k=5 122 either way).
     c.stage_lds = 6;
     c.unroll = 8;
     c.k_tile = 8;
     c.waves_per_block = 1;
     c.rows_per_lane = 1;
     c.xcd_remap = 1;
-    if (dtype != WK_F64) c.accumulate = WK_ACC_F64;
   }
   // as the launcher uses it (a masked last tile where the windows run it)
   c.k_tile = std::min(c.k_tile, masked ? pow2_at_least(std::max(1, k)) : pow2_at_most(std::max(1, k)));
