@@ -171,3 +171,26 @@ def test_fp32_default_sums_do_not_depend_on_the_size(nodes):
         eng.launch(dev(xq), other, cfg=dict(BASE, stage_lds=4, accumulate=capi.WK_ACC_TWOSUM))
         assert torch.equal(y, other), k
     eng.close()
+
+
+@pytest.mark.parametrize("dof,nodes,k,sets", [(2, 20800, 5, False), (2, 20800, 16, True), (2, 3200, 5, True),
+                                              (3, 44800, 8, False), (4, 11200, 5, True)])
+def test_default_on_short_block_rows(dof, nodes, k, sets):
+    """One dof x dof block a node, and two for dof 2: the row sets where they pay."""
+    say(f"[gpu] default, dof {dof}, {nodes} nodes, k={k}")
+    n, w = dof * nodes, 2 if dof == 2 else 1
+    node = np.arange(nodes)
+    nb = np.sort(np.stack([(node + i) % nodes for i in range(w)], 1), 1)
+    ci = np.repeat((nb[:, :, None] * dof + np.arange(dof)).reshape(nodes, -1), dof, 0).reshape(-1).astype(np.int32)
+    m = fe.CSR("short", n, n, (w * dof * np.arange(n + 1)).astype(np.int32), ci,
+               np.random.default_rng(1).uniform(-1, 1, ci.size))
+    x = fe.uniform_x(n, k, seed=9)
+    for dtype in ("f64", "f32"):
+        dt = np.float64 if dtype == "f64" else np.float32
+        v, xq = m.vals.astype(dt), x.astype(dt)
+        eng = engine(scan(m), m.vals, m.colind, dtype=dtype)
+        y = out(n, k)
+        got = ran(eng.launch, dev(xq), y, None)
+        assert bool(got & capi.WK_KERNEL_ROW_SETS) == sets, (dtype, got)
+        assert np.array_equal(y.cpu().numpy(), O.csr_spmv(m.rowptr, ci, v.astype(np.float64), xq.astype(np.float64)))
+        eng.close()

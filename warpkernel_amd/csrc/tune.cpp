@@ -48,6 +48,32 @@ int32_t default_sums(const DevLayout &D, int32_t k) {
   return D.rs_waves > 0 && k >= kRowSetColumns ? WK_ACC_F64 : WK_ACC_TWOSUM;
 }
 
+// Where the row sets beat the layout's other kernels, by the rows a wave sums (8
+// where sets hold two rows, 10 to 12 three, 16 four), the mean row length and
+// the groups.  Blocks of dof rows over a band of w nodes, d = dof, n = d w entries a
+// row, us by the other kernels and by the row sets:
+//   two rows a set, from 640 groups: short rows lose below k = 9 (3,750 groups, d 2:
+//   n 4 k=5 16.2 / 20.9, n 10 19.0 / 21.1, n 18 23.2 / 21.5; 936 groups, n 4 k=8 5.8 /
+//   6.7; 468 groups, n 4 k=8 4.0 / 3.9), and the shortest above (n 2 k=12 23.3 / 30.1,
+//   n 4 42.2 / 29.9); FP32 values with FP64 sums longer ones on large layouts
+//   (3,750 groups, n 18 k=5 15.7 / 18.7; 936 groups, n 6 5.8 / 5.8);
+//   three, large layouts: the shortest (3,750 groups, d 3: n 3 k=5 13.1 / 16.8, n 6 17.2 /
+//   16.8; FP32 n 3 10.5 / 14.6, n 6 14.3 / 14.6);
+//   up to three and fewer than 4 entries: k = 8, one tile of the direct kernel (249
+//   groups, d 3 n 3 2.6 / 2.8; 468 groups, d 2 n 2 3.0 / 3.8).
+// FP32 layouts of 8,192 groups or more keep the windows up to k = 8 (hex elasticity
+// 64^3 k=8 114 us against 126; k=5 122 either way).
+bool row_sets_pay(const DevLayout &D, int32_t dtype, int32_t k, double mean_len) {
+  const bool f64 = dtype == WK_F64;
+  const double rows = (double)D.nznrows / (double)D.rs_waves;
+  const bool two = rows < 10.0, three = rows < 14.0;  // at most
+  if (k >= 9) return !(two && mean_len < 4.0 && D.ngroups >= 640);
+  if (!f64 && D.ngroups >= 8192) return false;
+  if (k == 8 && three && mean_len < 4.0) return false;
+  if (two && D.ngroups >= 640 && mean_len < (f64 ? 12.0 : D.ngroups >= 2048 ? 24.0 : 6.0)) return false;
+  return !(three && D.ngroups >= 2048 && mean_len < (f64 ? 5.0 : 6.0));
+}
+
 // Candidate set: the knobs that change speed but not results.
 std::vector<wk_launch> candidates(const DevLayout &D, int32_t dtype, const wk_launch &base, int32_t k) {
   std::vector<wk_launch> out;
@@ -399,14 +425,12 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
     }
   }
   if (dtype != WK_F64) c.accumulate = sums != kDefaultSums ? sums : default_sums(D, k);
-  if (win_ok && row_sets_run(D, dtype, k, c.accumulate) && (dtype == WK_F64 || k >= 9 || D.ngroups < 8192)) {
+  if (win_ok && row_sets_run(D, dtype, k, c.accumulate) && row_sets_pay(D, dtype, k, mean_len)) {
     // row sets on the matrix cores (stage 6, rowsets.hip), all of k in one
     // launch.  Hex elasticity, FP64: 32^3 k=5 18.1 us against 36.4, k=8 18.7
     // against 30.9, k=16 25.1 against 58.4, k=32 38.4 against 100; 64^3 k=5
     // 176 against 194, k=8 181 against 204, k=16 248 against 421, k=32 382
-    // against 803.  FP32 values with FP64 sums: 32^3 k=8 13.7 us, 48^3 36.4;
-    // large layouts keep their windows up to k = 8 (64^3, 12,874 groups, k=8
-    // 114 us against 126; k=5 122 either way).
+    // against 803.  FP32 values with FP64 sums: 32^3 k=8 13.7 us, 48^3 36.4.
     c.stage_lds = 6;
     c.unroll = 8;
     c.k_tile = 8;
