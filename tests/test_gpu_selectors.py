@@ -194,3 +194,25 @@ def test_default_on_short_block_rows(dof, nodes, k, sets):
         assert bool(got & capi.WK_KERNEL_ROW_SETS) == sets, (dtype, got)
         assert np.array_equal(y.cpu().numpy(), O.csr_spmv(m.rowptr, ci, v.astype(np.float64), xq.astype(np.float64)))
         eng.close()
+
+
+@pytest.mark.parametrize("groups,lens,kernel", [
+    (1280, [39], capi.WK_KERNEL_PACKED), (313, [39], capi.WK_KERNEL_OFFSETS), (1280, [16], capi.WK_KERNEL_OFFSETS),
+    (2304, [20], capi.WK_KERNEL_PACKED), (1280, [1, 3, 9, 17, 33, 39], capi.WK_KERNEL_PACKED),
+    (1280, [1, 3, 9, 17], capi.WK_KERNEL_OFFSETS)])
+def test_default_on_bands(groups, lens, kernel):
+    """One right-hand side on bands of random columns: column offsets or x windows."""
+    say(f"[gpu] default on bands, {groups} groups, {lens}")
+    n = 64 * groups
+    rng = np.random.default_rng(3)
+    cnt = np.asarray(lens)[np.arange(n) % len(lens)]
+    rows = np.repeat(np.arange(n), cnt)
+    cols = np.clip(rows + rng.integers(-30, 31, rows.size), 0, n - 1)
+    ci = cols[np.lexsort((cols, rows))].astype(np.int32)
+    m = fe.CSR("band", n, n, np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32), ci, rng.uniform(-1, 1, ci.size))
+    x = fe.uniform_x(n, seed=2)
+    eng = engine(scan(m), m.vals, m.colind)
+    y = torch.full((n,), float("nan"), dtype=torch.float64, device="cuda")
+    assert ran(eng.launch, dev(x), y, None) == kernel
+    assert np.array_equal(y.cpu().numpy(), O.csr_spmv(m.rowptr, ci, m.vals, x))
+    eng.close()

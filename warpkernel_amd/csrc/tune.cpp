@@ -74,6 +74,35 @@ bool row_sets_pay(const DevLayout &D, int32_t dtype, int32_t k, double mean_len)
   return !(three && D.ngroups >= 2048 && mean_len < (f64 ? 5.0 : 6.0));
 }
 
+// One right-hand side: where x windows that pay (3 slots or more an entry) beat the
+// 16-bit column offsets, by mean row length, the longest group against it, the
+// groups, and reuse.  Few groups leave the windows' fill uncovered; long rows, and
+// long groups among short ones, take several of the offsets' batches, whose x
+// gathers the windows' LDS reads outrun.  us by offsets and by windows (bands of
+// random columns unless named; r: slots an entry):
+//   39 entries, FP64 1,000 groups 6.8 / 6.6, 1,563 9.8 / 8.2, 6,250 32.4 / 27.1;
+//     FP32 313 4.9 / 5.2, 1,000 6.6 / 6.0, 4,063 14.1 / 11.2, 9,375 r 4.0 32.8 / 27.0
+//   27 entries, FP64 1,563 6.6 / 6.6, 2,657 10.4 / 9.7; FP32 1,000 5.6 / 5.2, 4,063
+//     10.3 / 8.3, 9,375 r 4.0 23.5 / 20.9; hex diffusion r 3.0 to 3.4, FP64 48^3 (1,839) 7.2 / 7.6, 60^3 (3,547)
+//     13.6 / 12.7, 100^3 (16,098) 52.3 / 49.9, FP32 60^3 8.1 / 8.5, 100^3 29.9 / 33.3
+//   20 entries, FP64 2,032 6.3 / 6.8, 2,657 8.5 / 7.9; FP32 2,032 5.4 / 5.3, 2,657 6.5 / 5.4
+//   16 entries, FP64 4,063 9.5 / 9.9, 9,375 r 4.3 20.6 / 23.5, r 10 level
+//   1 to 39 entries, mean 17, FP64 858 7.1 / 7.1, 1,139 8.9 / 8.0, 4,018 24.9 / 23.3;
+//     FP32 737 6.3 / 5.1; 12 to 27, mean 18, FP64 2,032 8.2 / 8.4, 2,657 11.6 / 10.2, 9,375
+//     25.4 / 30.6; FP32 1,000 5.2 / 4.7, 9,375 19.3 / 21.1; 1 to 17, mean 7.5, 37.5 / 58.1
+bool windows_beat_offsets(const DevLayout &D, int32_t dtype, double mean_len, double reuse) {
+  const bool f64 = dtype == WK_F64;
+  const int32_t G = D.ngroups;
+  const double mix = (double)D.pk_longest / std::max(1.0, mean_len);
+  if (mean_len >= 32.0) return G >= (f64 ? 1280 : 768);
+  if (G >= 8192) return reuse >= (f64 ? 4.5 : 4.0) || (f64 && mean_len >= 20.0);
+  if (mean_len < 16.0) return false;
+  if (mix >= 1.8) return G >= (f64 ? 1024 : 512);
+  if (mix >= 1.4) return G >= (f64 ? 2304 : 768);
+  if (f64) return mean_len >= 20.0 && G >= 2304;
+  return reuse >= 4.0 && mean_len >= 20.0 && G >= (mean_len >= 24.0 ? 768 : 2304);
+}
+
 // Candidate set: the knobs that change speed but not results.
 std::vector<wk_launch> candidates(const DevLayout &D, int32_t dtype, const wk_launch &base, int32_t k) {
   std::vector<wk_launch> out;
@@ -215,11 +244,7 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
                               (D.variant == 2 && k >= 8 && reuse >= 2.5) ||
                               (dtype == WK_F64 && D.variant == 1 && k >= 4 && reuse >= 2.0 &&
                                mean_len < 20.0 && D.ngroups >= 4096));
-  // large layouts keep windows that are reused most (hex diffusion 100^3, 16,098
-  // groups, 3.4 slots per entry, 49.9 us against 52.3 by offsets; but 72^3, 6,079
-  // groups, 22.4 against 21.4, and FP32 100^3 33.3 against 29.9)
-  const bool keep_windows =
-      windows && D.ngroups >= 8192 && (reuse >= 4.5 || (dtype == WK_F64 && mean_len >= 20.0));
+  const bool keep_windows = windows && windows_beat_offsets(D, dtype, mean_len, reuse);
   if (k == 1 && !kr && D.dl_words && win_ok && D.nd_max == 0 && !keep_windows) {
     // 16-bit column offsets (deltas.hip).  P1 tets 96^3 30.4 -> 27.8 us (FP32
     // 23.9 -> 18.8), 60^3 9.5 -> 7.5; large layouts without the remap (96^3 27.8
