@@ -171,7 +171,7 @@ namespace {
 // Copies one host layout (and its padded values/columns) to the device.
 // vals/colind are the layout's own CSR; slot_of_nz (optional) replaces
 // reorder_rows as the map from A's CSR order to slots (the row sort and the
-// transpose, whose slots then take their CSR entries one by one).
+// transpose, whose slots take their CSR entries one by one where few are pads).
 void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double *vals,
                    const int32_t *colind, int32_t dtype, bool kr, const uint32_t *slot_of_nz,
                    hipStream_t s) {
@@ -210,7 +210,8 @@ void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double 
     D.row_off = dev_upload(E, L.row_offset_warp.data(), (int64_t)L.row_offset_warp.size(), s);
   }
   std::vector<int32_t> src;
-  if (&D == &E->adj) {
+  for (uint32_t n : D.h_max_nz_rows) D.longest = std::max(D.longest, n);
+  if (&D == &E->adj && L.allocate_nz <= kGatherPads * L.nz) {
     src.assign((size_t)L.allocate_nz, -1);
     for (int64_t i = 0; i < L.nz; i++) src[slot_of_nz[i]] = (int32_t)i;
     D.src_of_slot = dev_upload(E, src.data(), (int64_t)src.size(), s);

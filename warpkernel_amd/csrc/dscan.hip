@@ -664,6 +664,7 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
 
   // 5. x windows, when every group fits
   const uint32_t longest = G ? *std::max_element(A.begin(), A.end()) : 0;
+  D.longest = longest;
   const bool windows = G && (int64_t)longest * 64 <= kWinSlots;
   // the uploads' host arrays go, and the caller may use the engine on another
   // stream or free the CSR (with windows, their counts' download waits)

@@ -3,15 +3,16 @@
 // alone, on the device.
 //
 // Layouts whose lanes hold runs of CSR entries (every forward layout without
-// the row sort): one block per group reads its rows' entries 4 to 64 at a time,
-// turns them around in LDS and writes whole steps.  It streams 16 bytes per
-// FP64 entry, both ways in whole lines, with no index array.  (One thread per
-// entry writing through the CSR-to-slot map put 8 bytes into each 128-byte
-// line: hex elasticity 48^3, 27.4M entries, 305 us against 77.)  The
-// transposed layout reads the entry of each slot instead: indices and values
-// written in order, the 8-byte reads land on lines that the same group's other
-// steps read too (hex diffusion 48^3, both layouts 31 us as two scatters,
-// 23 here in one launch).
+// the row sort) and whose longest group is no bottleneck: one block per group
+// reads its rows' entries 4 to 64 at a time, turns them around in LDS and writes
+// whole steps.  It streams 16 bytes per FP64 entry, both ways in whole lines,
+// with no index array.  (One thread per entry writing through the CSR-to-slot map
+// put 8 bytes into each 128-byte line: hex elasticity 48^3, 27.4M entries, 305 us
+// against 77.)  The transposed layout, unless padded much, reads the entry of each
+// slot instead: indices and values written in order, the 8-byte reads land on
+// lines that the same group's other steps read too (hex diffusion 48^3, both
+// layouts 31 us as two scatters, 23 here in one launch).  The others go through
+// the map.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -103,7 +104,8 @@ __global__ __launch_bounds__(TH) void update_kernel(UpdateArgs u) {
     gather_slots<T, TH>(u, work_id(b - u.ngroups, u.nblocks_t, 1));
 }
 
-// Row-sorted layouts, whose lanes hold no runs: entry i to slot[i].
+// Layouts whose lanes hold no runs (the row sort), with a group much longer than
+// its share of the entries, or padded much: entry i to slot[i].
 template <class T>
 __global__ __launch_bounds__(kThreads) void scatter_kernel(const T *__restrict__ src,
                                                            const uint32_t *__restrict__ slot,
@@ -113,24 +115,21 @@ __global__ __launch_bounds__(kThreads) void scatter_kernel(const T *__restrict__
     dst[slot[i]] = src[i];
 }
 
+// Entry i of the CSR to slot[i].
+template <class T>
+void scatter(const DevLayout &D, const void *vals, int64_t nnz, hipStream_t s) {
+  if (!D.slot_of_nz) fail(WK_ERR_STATE, "layout has no device scatter map");
+  const int64_t blocks = std::min<int64_t>((nnz + kThreads - 1) / kThreads, 65536);
+  hipLaunchKernelGGL(scatter_kernel<T>, dim3((uint32_t)blocks), dim3(kThreads), 0, s,
+                     static_cast<const T *>(vals), D.slot_of_nz, static_cast<T *>(D.vals), nnz);
+  hip_check(hipGetLastError(), "scatter launch");
+}
+
 template <class T>
 void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
   const DevLayout &D = E->fwd;
   UpdateArgs u{};
   u.src = vals;
-  if (D.lane_src) {
-    u.dst = D.vals;
-    u.lane_src = reinterpret_cast<const int2 *>(D.lane_src);
-    u.warp_offsets = D.warp_offsets;
-    u.max_nz_rows = D.max_nz_rows;
-    u.ngroups = D.ngroups;
-  } else {
-    if (!D.slot_of_nz) fail(WK_ERR_STATE, "layout has no device scatter map");
-    const int64_t blocks = std::min<int64_t>((E->nnz + kThreads - 1) / kThreads, 65536);
-    hipLaunchKernelGGL(scatter_kernel<T>, dim3((uint32_t)blocks), dim3(kThreads), 0, s,
-                       static_cast<const T *>(vals), D.slot_of_nz, static_cast<T *>(D.vals), E->nnz);
-    hip_check(hipGetLastError(), "scatter launch");
-  }
   // The steps turned at a time, by mean row length.  Up to 4 and 8, where there are
   // groups enough, one wave a group: most of a 16-step tile and three of its waves
   // would be empty (threshold 5, P1 tets 54^3, 10,399 groups, 14.1 -> 8.5 us, 9.6 by
@@ -150,11 +149,28 @@ void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
                     : sizeof(T) == 4 || D.allocate_nz <= 32 * slots ? 32
                                                                     : 64;
   const int threads = steps <= 8 ? 64 : steps == 64 ? 512 : kThreads;
-  if (E->has_adj) {
+  // A block turns its group's steps one tile after another, 0.7 to 1.5 us each,
+  // while the map takes 11 us per million FP64 entries, 6 per million FP32 ones,
+  // whatever the rows: layouts with a group too long for its share keep the map
+  // (200,000 rows of 9 entries and one of 100,000: 9.8 us, 1,568 turned; 64 of 8,000
+  // 13.6, 419; 1,500 rows of 1,500, 24 groups, 25.4, 39.2; but 20,000 of 500 147, 37.9)
+  const int64_t turns = ((int64_t)D.longest + steps - 1) / steps;
+  if (D.lane_src && turns <= 3 + E->nnz / (sizeof(T) == 8 ? 131072 : 262144)) {
+    u.dst = D.vals;
+    u.lane_src = reinterpret_cast<const int2 *>(D.lane_src);
+    u.warp_offsets = D.warp_offsets;
+    u.max_nz_rows = D.max_nz_rows;
+    u.ngroups = D.ngroups;
+  } else {
+    scatter<T>(D, vals, E->nnz, s);
+  }
+  if (E->has_adj && E->adj.src_of_slot) {
     u.dst_t = E->adj.vals;
     u.src_of_slot = E->adj.src_of_slot;
     u.slots_t = E->adj.allocate_nz;
     u.nblocks_t = (int32_t)((u.slots_t + threads * kGatherPer - 1) / (threads * kGatherPer));
+  } else if (E->has_adj) {
+    scatter<T>(E->adj, vals, E->nnz, s);
   }
   const int64_t blocks = (int64_t)u.ngroups + u.nblocks_t;
   if (blocks > INT32_MAX) fail(WK_ERR_LIMIT, "grid too large");
