@@ -130,7 +130,11 @@ class device_vector {
   void resize(size_t n) {
     if (n == n_) return;
     release();
-    if (n) hip_check(hipMalloc(reinterpret_cast<void **>(&p_), n * sizeof(T)));
+    if (n && hipMalloc(reinterpret_cast<void **>(&p_), n * sizeof(T)) != hipSuccess) {
+      (void)hipGetLastError();
+      wk_release_memory();  // memory of destroyed engines
+      hip_check(hipMalloc(reinterpret_cast<void **>(&p_), n * sizeof(T)));
+    }
     n_ = n;
   }
   void resize_fill(size_t n, T fill) { assign(std::vector<T>(n, fill)); }

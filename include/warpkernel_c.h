@@ -261,6 +261,13 @@ int wk_engine_create_device(int32_t variant, int32_t threshold, int32_t max_tpr,
                             const int32_t *colind_dev, const double *vals_dev,
                             int32_t values_dtype, uint32_t flags, void *stream, wk_engine **out);
 
+/* Device memory of destroyed engines, of which the library keeps up to 2 GiB per
+ * device for the next engines: all of it goes back to the devices, for other
+ * allocators of the process.  Returns the bytes.  (The library's own allocations
+ * take it back before they fail.)  Any thread may call it at any time outside
+ * graph capture. */
+int64_t wk_release_memory(void);
+
 /* engine arrays (wk_engine_download), besides WK_ROW_MAP .. WK_ROW_OFFSET_WARP
  * (WK_REORDER_ROWS gives the CSR-to-slot map; WK_ROW_MAP_INV exists for
  * engines built by wk_engine_create_device) */

@@ -83,6 +83,7 @@ SIGNATURES = {
     "wk_scatter": (C.c_int, [P, P, P, I64, I64, I32, P]),
     "wk_engine_create": (C.c_int, [P, P, P, P, I32, U32, P, PP]),
     "wk_engine_destroy": (None, [P]),
+    "wk_release_memory": (I64, []),
     "wk_engine_get_info": (C.c_int, [P, C.POINTER(LayoutInfo)]),
     "wk_engine_update_values": (C.c_int, [P, P, P]),
     "wk_engine_set_colinds": (C.c_int, [P, P, I32, P]),

@@ -490,6 +490,13 @@ class engine:
             pass
 
 
+def release_memory() -> int:
+    """Gives the device memory of destroyed engines, of which the library keeps up
+    to 2 GiB per device for the next ones, back to the devices (for torch, say).
+    Returns the bytes."""
+    return int(lib().wk_release_memory())
+
+
 class _EngineLayout:
     """The layout of an engine scanned on the device: structure's scalars, and
     its arrays downloaded on first use (kept with the engine)."""

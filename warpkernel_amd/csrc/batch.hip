@@ -368,7 +368,7 @@ int wk_batch_create(wk_engine *const *engines, int32_t count, int32_t waves_per_
       hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, B->device), "attr");
       B->nwaves = waves_per_cu ? cus * waves_per_cu : 0;
       B->desc.resize(count);
-      hip_check(hipMalloc(&B->d_desc, sizeof(BatchDesc) * count), "hipMalloc");
+      B->d_desc = static_cast<BatchDesc *>(device_malloc(sizeof(BatchDesc) * count));
       // the work list has one item per group and per 64 rows without nonzeros
       // of every engine, whatever the bound vectors and k
       int64_t nitems = 0;
@@ -376,9 +376,9 @@ int wk_batch_create(wk_engine *const *engines, int32_t count, int32_t waves_per_
         nitems += (int64_t)E->fwd.ngroups + (E->fwd.nrows - E->fwd.nznrows + 63) / 64;
       if (nitems > (int64_t)INT32_MAX) fail(WK_ERR_LIMIT, "too many work items");
       B->nitems = nitems;
-      if (nitems) hip_check(hipMalloc(&B->d_items, sizeof(BatchItem) * (size_t)nitems), "hipMalloc");
+      if (nitems) B->d_items = static_cast<BatchItem *>(device_malloc(sizeof(BatchItem) * (size_t)nitems));
       if (B->nwaves) {
-        hip_check(hipMalloc(&B->d_wstart, sizeof(int32_t) * (B->nwaves + 1)), "hipMalloc");
+        B->d_wstart = static_cast<int32_t *>(device_malloc(sizeof(int32_t) * (B->nwaves + 1)));
       }
     } catch (...) {
       free_batch(B);

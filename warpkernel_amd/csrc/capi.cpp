@@ -35,7 +35,8 @@ namespace {
 // unmapping and clearing each time: hex elasticity 40^3, 0.5 GB in 25 blocks,
 // 1.1 ms to build and 1.7 to 8.2 ms to free.  Bounded to kKeepBytes per device
 // (0.7% of its memory), given back to the device from the oldest on when the
-// bound is passed, and all of it when an allocation fails.
+// bound is passed, and all of it when an allocation of this library fails or the
+// program asks (wk_release_memory), since another allocator in the process cannot.
 constexpr size_t kKeepBytes = size_t(2) << 30;
 constexpr size_t kKeepLeast = size_t(256) << 10;  // smaller blocks cost nothing to allocate
 
@@ -78,17 +79,28 @@ void *block_take(size_t &bytes) {
       return p;
     }
   }
+  return device_malloc(bytes);
+}
+
+void *device_malloc(size_t bytes) {
   void *p = nullptr;
   if (hipMalloc(&p, bytes) == hipSuccess) return p;
   (void)hipGetLastError();
+  blocks_release();
+  hip_check(hipMalloc(&p, bytes), "hipMalloc");
+  return p;
+}
+
+int64_t blocks_release() noexcept {
   std::vector<KeptBlock> all;
   {
     std::lock_guard<std::mutex> g(g_kept_mu);
     all.swap(g_kept);
   }
-  free_blocks(all);
-  hip_check(hipMalloc(&p, bytes), "hipMalloc");
-  return p;
+  int64_t bytes = 0;
+  for (const KeptBlock &k : all) bytes += (int64_t)k.bytes;
+  if (!all.empty()) free_blocks(all);
+  return bytes;
 }
 
 void block_give(int device, void *p, size_t bytes) noexcept {
@@ -545,6 +557,8 @@ int wk_engine_create(const wk_layout *L, const int32_t *rowptr_host, const int32
 
 void wk_engine_destroy(wk_engine *E) { free_engine(E); }
 
+int64_t wk_release_memory(void) { return blocks_release(); }
+
 int wk_engine_get_info(const wk_engine *E, wk_layout_info *info) {
   return guarded([&] {
     check_engine(E);
@@ -574,7 +588,7 @@ int wk_engine_set_colinds(wk_engine *E, const int32_t *pcols, int32_t where, voi
         if (p) (void)hipFree(p);
       }
     } flags;
-    hip_check(hipMalloc(reinterpret_cast<void **>(&flags.p), sizeof(int32_t) * kColFlags), "hipMalloc");
+    flags.p = static_cast<int32_t *>(device_malloc(sizeof(int32_t) * kColFlags));
     swap_colinds(E, pcols, where, static_cast<hipStream_t>(stream), flags.p);
   });
 }

@@ -330,6 +330,10 @@ int guarded(F &&f) {
 // nothing on the device may still use them.
 void *block_take(size_t &bytes);
 void block_give(int device, void *p, size_t bytes) noexcept;
+// Gives the kept blocks back to their devices; how many bytes they were.
+int64_t blocks_release() noexcept;
+// hipMalloc that gives the kept blocks back before it fails.
+void *device_malloc(size_t bytes);
 
 // Device allocations owned (and given back) by an engine.
 template <class T>
