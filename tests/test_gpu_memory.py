@@ -74,3 +74,34 @@ def test_release_beside_living_engines():
     assert torch.equal(y[0], y[1]) and torch.equal(y[0], y[2])
     bt.close()
     a.close()
+
+
+@pytest.mark.parametrize("where", ["host", "device"])
+def test_offsets_that_do_not_fit_are_given_back(where):
+    """A band of 2M rows of 5 entries: its column offsets take 32 MB, which an
+    engine keeps only if every one of them fits 16 bits."""
+    say(f"[gpu] memory of offsets that do not fit, {where}")
+    n = 2_000_000
+    used = []
+    for far in (0, 1):
+        rows = np.arange(n, dtype=np.int32)
+        ci = np.clip(rows[:, None] + np.arange(-2, 3, dtype=np.int32), 0, n - 1).astype(np.int32)
+        if far:
+            ci[n // 2, 0] = 7  # a million columns off the diagonal
+        rp, vals = (5 * np.arange(n + 1)).astype(np.int32), np.ones(5 * n)
+        csr = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (rp, ci.reshape(-1), vals)]
+        gc.collect()
+        warpkernel_amd.release_memory()
+        start = free()
+        if where == "host":
+            s = structure(64).scan(5 * n, n, vals, rp, ci.reshape(-1))
+            eng = engine(s, vals, ci.reshape(-1))
+        else:
+            eng = engine.from_device(*csr)
+        warpkernel_amd.release_memory()
+        used.append(start - free())
+        x, y = torch.ones(n, dtype=torch.float64, device="cuda"), torch.empty(n, dtype=torch.float64, device="cuda")
+        eng.launch(x, y)
+        assert bool((y == 5).all())
+        eng.close()
+    assert used[0] - used[1] > 24 * MIB, used

@@ -174,7 +174,7 @@ void build_compact_columns(wk_engine *E, DevLayout &D, uint32_t *scratch, hipStr
   hip_check(hipMemcpyAsync(h.data(), scratch, 4 * words, hipMemcpyDeviceToHost, stream), "compact columns");
   hip_check(hipStreamSynchronize(stream), "compact columns");
   const uint32_t *hw = reinterpret_cast<const uint32_t *>(h.data());
-  if (offsets) deltas_finish(D, hw + 3 * G + 1);
+  if (offsets) deltas_finish(E, D, hw + 3 * G + 1);
   if (sets) row_sets_finish(E, D, starts, span, h.data(), hw + 2 * G, stream);
 }
 

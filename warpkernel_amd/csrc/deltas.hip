@@ -169,7 +169,7 @@ bool launch_deltas(const DevLayout &D, int prec, int out, const SpmvArgs &a, int
 }
 
 // The words do not depend on whether they fit, so they are written at once and
-// dropped by the caller (deltas_finish false) if some group's do not.
+// given back by deltas_finish if some group's do not.
 bool deltas_begin(wk_engine *E, DevLayout &D, std::vector<uint32_t> &off, uint32_t *fits, uint32_t *dev_off,
                   hipStream_t stream) {
   const int32_t G = D.ngroups;
@@ -195,9 +195,10 @@ bool deltas_begin(wk_engine *E, DevLayout &D, std::vector<uint32_t> &off, uint32
   return true;
 }
 
-void deltas_finish(DevLayout &D, const uint32_t *fits) {
+void deltas_finish(wk_engine *E, DevLayout &D, const uint32_t *fits) {
   for (int32_t g = 0; g < D.ngroups; g++)
     if (!fits[g]) {
+      dev_give(E, D.dl_words);
       D.dl_words = nullptr;
       D.dl_off = nullptr;
       return;

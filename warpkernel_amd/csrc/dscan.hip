@@ -711,8 +711,7 @@ void device_scan(wk_engine *E, int32_t variant, int32_t threshold, int32_t max_t
       taken.idle = true;
       build_compact_columns(E, D, reinterpret_cast<uint32_t *>(dcount), s);
     } else {
-      block_give(E->device, E->owned.back().first, E->owned.back().second);  // idx
-      E->owned.pop_back();
+      dev_give(E, idx);
     }
   }
 

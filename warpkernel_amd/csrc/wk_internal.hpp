@@ -244,11 +244,11 @@ void build_compact_columns(wk_engine *E, DevLayout &D, uint32_t *scratch, hipStr
 bool row_sets_begin(DevLayout &D, uint64_t *starts, uint32_t *span, hipStream_t stream);
 void row_sets_finish(wk_engine *E, DevLayout &D, const uint64_t *starts, uint32_t *span, const uint64_t *hs,
                      const uint32_t *hw, hipStream_t stream);
-// Offsets: fits [ngroups] on the device, downloaded for finish; off stays alive
-// until then, dev_off [ngroups + 1] as long as the engine.
+// Offsets: fits [ngroups] on the device, downloaded for finish (nothing uses the
+// words then); off stays alive until then, dev_off [ngroups + 1] as long as the engine.
 bool deltas_begin(wk_engine *E, DevLayout &D, std::vector<uint32_t> &off, uint32_t *fits, uint32_t *dev_off,
                   hipStream_t stream);
-void deltas_finish(DevLayout &D, const uint32_t *fits);
+void deltas_finish(wk_engine *E, DevLayout &D, const uint32_t *fits);
 // Right-hand sides from which the row sets run: below, the windows read less (hex
 // elasticity 64^3 k=4 118 us against 175; 32^3 17.5 either way).
 constexpr int32_t kRowSetColumns = 5;
@@ -343,6 +343,16 @@ T *dev_alloc(wk_engine *E, int64_t count) {
   void *p = block_take(bytes);
   E->owned.push_back({p, bytes});
   return static_cast<T *>(p);
+}
+
+// Gives one of them back ahead of the engine; nothing on the device uses it.
+inline void dev_give(wk_engine *E, const void *p) {
+  for (size_t i = 0; i < E->owned.size(); i++)
+    if (E->owned[i].first == p) {
+      block_give(E->device, E->owned[i].first, E->owned[i].second);
+      E->owned.erase(E->owned.begin() + (std::ptrdiff_t)i);
+      return;
+    }
 }
 
 template <class T>
