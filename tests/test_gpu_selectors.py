@@ -216,3 +216,23 @@ def test_default_on_bands(groups, lens, kernel):
     assert ran(eng.launch, dev(x), y, None) == kernel
     assert np.array_equal(y.cpu().numpy(), O.csr_spmv(m.rowptr, ci, m.vals, x))
     eng.close()
+
+
+def test_default_where_row_sets_do_not_reach():
+    """x as eight columns of an array of more than 4 GiB: the windows' choice."""
+    say("[gpu] default on columns of a wide array")
+    m = fe.hex_elastic_3d(7)
+    k = 8
+    x = fe.uniform_x(m.ncols, k, seed=3)
+    eng = engine(scan(m), m.vals, m.colind)
+    wide = torch.empty((m.ncols, (1 << 32) // (8 * m.ncols) + 1), dtype=torch.float64, device="cuda")
+    wide[:, 5:5 + k] = dev(x)
+    near = torch.empty((m.ncols, 2 * k), dtype=torch.float64, device="cuda")
+    near[:, :k] = dev(x)
+    ref = O.csr_spmv(m.rowptr, m.colind, m.vals, x)
+    for xd, sets in ((wide[:, 5:5 + k], False), (near[:, :k], True)):
+        y = out(m.nrows, k)
+        got = ran(eng.launch, xd, y, None)
+        assert got == capi.WK_KERNEL_ROW_SETS if sets else windows(got), got
+        assert np.array_equal(y.cpu().numpy(), ref)
+    eng.close()

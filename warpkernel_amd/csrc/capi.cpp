@@ -263,8 +263,8 @@ void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double 
   }
 }
 
-wk_launch resolve(wk_engine *E, int32_t op, int32_t k, const wk_launch *cfg) {
-  return cfg ? *cfg : engine_launch(E, op, k);
+wk_launch resolve(wk_engine *E, int32_t op, int32_t k, const wk_launch *cfg, int64_t ldx = 1) {
+  return cfg ? *cfg : engine_launch(E, op, k, kDefaultSums, ldx);
 }
 
 void check_engine(const wk_engine *E) {
@@ -632,7 +632,7 @@ int wk_run(wk_engine *E, const wk_launch *cfg, const void *x_dev, double *y_dev,
     check_engine(E);
     if ((!x_dev && E->ncols) || (!y_dev && E->nrows)) fail(WK_ERR_ARG, "NULL vector");
     if (ldx < k || ldy < k) fail(WK_ERR_ARG, "leading dimension smaller than k");
-    launch_spmv(E->fwd, E->dtype, resolve(E, WK_OP_RUN, k, cfg), OUT_RUN, x_dev, ldx, y_dev, ldy, nullptr, 0, k,
+    launch_spmv(E->fwd, E->dtype, resolve(E, WK_OP_RUN, k, cfg, ldx), OUT_RUN, x_dev, ldx, y_dev, ldy, nullptr, 0, k,
                 static_cast<hipStream_t>(stream));
   });
 }
@@ -644,7 +644,7 @@ int wk_run_x(wk_engine *E, const wk_launch *cfg, const void *x_dev, double *y_de
     if (E->nrows != E->ncols) fail(WK_ERR_ARG, "the Kr form needs a square matrix");
     if ((!x_dev && E->ncols) || (!y_dev && E->nrows)) fail(WK_ERR_ARG, "NULL vector");
     if (ldx < k || ldy < k) fail(WK_ERR_ARG, "leading dimension smaller than k");
-    launch_spmv(E->fwd, E->dtype, resolve(E, WK_OP_RUN_X, k, cfg), OUT_RUNX, x_dev, ldx, y_dev, ldy, nullptr, 0, k,
+    launch_spmv(E->fwd, E->dtype, resolve(E, WK_OP_RUN_X, k, cfg, ldx), OUT_RUNX, x_dev, ldx, y_dev, ldy, nullptr, 0, k,
                 static_cast<hipStream_t>(stream));
   });
 }
@@ -657,7 +657,7 @@ int wk_residual(wk_engine *E, const wk_launch *cfg, const double *b_dev, int64_t
     if (E->dtype != WK_F64) fail(WK_ERR_ARG, "the residual is computed by FP64 engines");
     if ((!x_dev && E->ncols) || ((!r_dev || !b_dev) && E->nrows)) fail(WK_ERR_ARG, "NULL vector");
     if (ldx < k || ldr < k || ldb < k) fail(WK_ERR_ARG, "leading dimension smaller than k");
-    launch_spmv(E->fwd, E->dtype, resolve(E, WK_OP_RUN, k, cfg), OUT_RESID, x_dev, ldx, r_dev, ldr, b_dev, ldb, k,
+    launch_spmv(E->fwd, E->dtype, resolve(E, WK_OP_RUN, k, cfg, ldx), OUT_RESID, x_dev, ldx, r_dev, ldr, b_dev, ldb, k,
                 static_cast<hipStream_t>(stream));
   });
 }
@@ -669,7 +669,7 @@ int wk_run_adjoint(wk_engine *E, const wk_launch *cfg, const void *dy_dev, doubl
     if (!E->has_adj) fail(WK_ERR_STATE, "engine was created without WK_ENGINE_ADJOINT");
     if ((!dy_dev && E->nrows) || (!dx_dev && E->ncols)) fail(WK_ERR_ARG, "NULL vector");
     if (lddy < k || lddx < k) fail(WK_ERR_ARG, "leading dimension smaller than k");
-    launch_spmv(E->adj, E->dtype, resolve(E, WK_OP_ADJOINT, k, cfg), OUT_RUN, dy_dev, lddy, dx_dev, lddx, nullptr, 0,
+    launch_spmv(E->adj, E->dtype, resolve(E, WK_OP_ADJOINT, k, cfg, lddy), OUT_RUN, dy_dev, lddy, dx_dev, lddx, nullptr, 0,
                 k, static_cast<hipStream_t>(stream));
   });
 }
@@ -706,7 +706,7 @@ int wk_backward(wk_engine *E, const wk_launch *cfg, const void *dy_dev, int64_t 
                       E->d_tile_row, E->nnz, static_cast<const double *>(x_dev), dvals_dev, s);
       return;
     }
-    const wk_launch c = resolve(E, WK_OP_ADJOINT, k, cfg);
+    const wk_launch c = resolve(E, WK_OP_ADJOINT, k, cfg, lddy);
     launch_spmv(E->adj, E->dtype, c, OUT_RUN, dy_dev, lddy, dx_dev, lddx, nullptr, 0, k, s);
     launch_dvals(E->d_rowptr, E->d_colind, E->d_tile_row, E->d_rowind, E->nnz,
                  static_cast<const double *>(dy_dev), lddy, static_cast<const double *>(x_dev), ldx,

@@ -375,8 +375,7 @@ bool launch_rowsets(const DevLayout &D, int prec, int out, const SpmvArgs &a0, i
   const bool kr = out == OUT_RUNX;
   if (!D.rs_waves || D.win_max <= 0 || prec == 1 || k < kRowSetColumns || (kr && !D.rs_cols_kr)) return false;
   SpmvArgs a = a0;
-  const int64_t xsz = prec == 0 ? 8 : 4;
-  if ((int64_t)D.ncols * a.ldx * xsz > (int64_t)UINT32_MAX) return false;  // 32-bit offsets into x
+  if (!row_sets_reach(D, prec == 0 ? WK_F64 : WK_F32, a.ldx)) return false;
   // Tiles of 8 or 16 columns.  The widest that k fills: it costs one pass
   // over a wave's columns, and 16 FP64 values are a whole 128-byte line of x
   // (hex elasticity 64^3 k=32, 16-column tiles 382 us, 8-column ones 506).

@@ -217,7 +217,7 @@ std::vector<wk_launch> candidates(const DevLayout &D, int32_t dtype, const wk_la
 
 }  // namespace
 
-wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr, int32_t sums) {
+wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr, int32_t sums, int64_t ldx) {
   wk_launch c;
   wk_launch_default(&c);
   bool masked = false;  // k-tiles may exceed k (windowed multi-RHS)
@@ -450,7 +450,8 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
     }
   }
   if (dtype != WK_F64) c.accumulate = sums != kDefaultSums ? sums : default_sums(D, k);
-  if (win_ok && row_sets_run(D, dtype, k, c.accumulate) && row_sets_pay(D, dtype, k, mean_len)) {
+  if (win_ok && row_sets_run(D, dtype, k, c.accumulate) && row_sets_pay(D, dtype, k, mean_len) &&
+      row_sets_reach(D, dtype, ldx)) {
     // row sets on the matrix cores (stage 6, rowsets.hip), all of k in one
     // launch.  Hex elasticity, FP64: 32^3 k=5 18.1 us against 36.4, k=8 18.7
     // against 30.9, k=16 25.1 against 58.4, k=32 38.4 against 100; 64^3 k=5
@@ -468,7 +469,7 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
   return c;
 }
 
-wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k, int32_t sums) {
+wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k, int32_t sums, int64_t ldx) {
   const DevLayout &D = layout_for(E, op);
   {
     std::lock_guard<std::mutex> g(E->cfg_mu);
@@ -482,7 +483,7 @@ wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k, int32_t sums) {
       }
     }
   }
-  return heuristic_launch(D, E->dtype, k, op == WK_OP_RUN_X, sums);
+  return heuristic_launch(D, E->dtype, k, op == WK_OP_RUN_X, sums, ldx);
 }
 
 }  // namespace wk

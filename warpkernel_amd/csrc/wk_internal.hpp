@@ -252,6 +252,10 @@ void deltas_finish(wk_engine *E, DevLayout &D, const uint32_t *fits);
 // Right-hand sides from which the row sets run: below, the windows read less (hex
 // elasticity 64^3 k=4 118 us against 175; 32^3 17.5 either way).
 constexpr int32_t kRowSetColumns = 5;
+// Whether their 32-bit byte offsets reach every x (columns of an array of ldx).
+inline bool row_sets_reach(const DevLayout &D, int32_t dtype, int64_t ldx) {
+  return ldx <= (int64_t)UINT32_MAX / (dtype == WK_F64 ? 8 : 4) / (D.ncols > 0 ? D.ncols : 1);
+}
 // k right-hand sides through the row sets.  prec: 0 FP64, 2 FP32 values with
 // FP64 accumulation.  Returns false, nothing launched, where the layout or the
 // vectors do not allow it.
@@ -296,8 +300,11 @@ int64_t dvals_tile_size();
 // layout's choice for those sums: hex elasticity 32^3 k=8 compensated 24.1 us
 // against 31.3 with the row sets' other fields, 48^3 k=32 256 against 357).
 constexpr int32_t kDefaultSums = -1;
-wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k, int32_t sums = kDefaultSums);
-wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr, int32_t sums);
+// ldx: of the vectors to come, or 0 for any that the row sets reach (x as columns
+// of an array of more than 4 GiB keeps the windows' choice, hex elasticity 64^3 k=8
+// 204 us, where stage 6 would run the register kernel, 236).
+wk_launch engine_launch(wk_engine *E, int32_t op, int32_t k, int32_t sums = kDefaultSums, int64_t ldx = 0);
+wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr, int32_t sums, int64_t ldx);
 
 // WPK2's group split (warpkernel.hpp:633-691) over the longest row of each
 // W-row group of sorted rows (aw0); nzr = non-empty rows.  Outputs per
