@@ -236,3 +236,25 @@ def test_default_where_row_sets_do_not_reach():
         assert got == capi.WK_KERNEL_ROW_SETS if sets else windows(got), got
         assert np.array_equal(y.cpu().numpy(), ref)
     eng.close()
+
+
+def test_layouts_that_have_offsets_and_row_sets():
+    """The layouts of test_gpu_deltas and test_gpu_rowsets hold what they are there
+    for, also where the rows do not fill the last group."""
+    say("[gpu] offsets and row sets are there")
+    from test_gpu_deltas import CASES as BANDS
+    from test_gpu_rowsets import CASES as BLOCKS
+    for name, make in BANDS.items():
+        m = make()
+        eng = engine(scan(m), m.vals, m.colind)
+        y = torch.empty(m.nrows, dtype=torch.float64, device="cuda")
+        want = capi.WK_KERNEL_DIRECT if name == "too_wide" else capi.WK_KERNEL_OFFSETS
+        assert ran(eng.launch, dev(fe.uniform_x(m.ncols)), y, dict(BASE, k_tile=1, stage_lds=0)) == want, name
+        eng.close()
+    for name, make in BLOCKS.items():
+        m = make()
+        eng = engine(scan(m), m.vals, m.colind)
+        got = ran(eng.launch, dev(fe.uniform_x(m.ncols, 8)), out(m.nrows, 8), dict(BASE, stage_lds=6))
+        say(name, got)
+        assert (got == capi.WK_KERNEL_ROW_SETS) == (name != "long"), (name, got)
+        eng.close()

@@ -415,7 +415,9 @@ void row_sets_finish(wk_engine *E, DevLayout &D, const uint64_t *starts, uint32_
   uint32_t widest = 0;
   int most = 0;  // waves of one group
   for (int32_t g = 0; g < G; g++) {
-    const int n = __builtin_popcountll(hs[g]);
+    // (lanes past the last row hold no set)
+    const int32_t rows = std::min(64, D.nznrows - 64 * g);
+    const int n = __builtin_popcountll(hs[g] & (~0ull >> (64 - rows)));
     sets += n;
     waves += (n + 3) / 4;
     most = std::max(most, (n + 3) / 4);
