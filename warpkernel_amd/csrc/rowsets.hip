@@ -142,9 +142,14 @@ __device__ __forceinline__ void rowset_wave(const SpmvArgs &a, const SetRec *rec
       double bv[E];
 #pragma unroll
       for (int e = 0; e < E; e++) bv[e] = br[e];
+      if (others <= 0) {
 #pragma unroll
-      for (int e = 0; e < E; e++)
-        if (e >= others) yr[e] = bv[e] - acc[e];
+        for (int e = 0; e < E; e++) yr[e] = bv[e] - acc[e];
+      } else {
+#pragma unroll
+        for (int e = 1; e < E; e++)
+          if (e >= others) yr[e] = bv[e] - acc[e];
+      }
     } else {
 #pragma unroll
       for (int e = 0; e < E; e++) yr[e] = acc[e];
@@ -156,7 +161,10 @@ __device__ __forceinline__ void rowset_wave(const SpmvArgs &a, const SetRec *rec
 #pragma unroll
   for (int s = 0; s < KS; s++) av[s] = s < KS - CS || 4 * s + k4 < len ? (double)raw[s] : -0.0;
   int32_t t = 0;
-  for (; t + 1 < ntiles; t++) {
+  // (tiles of 4 and 8 columns come alone, launch_rowsets: without the loop the
+  // residual's kernel for 5 to 8 columns does not spill, blocks of
+  // three unknowns on 56^3 nodes k=8 164 -> 130 us)
+  for (; (E == 4 || OUT != OUT_RESID) && t + 1 < ntiles; t++) {
     const uint32_t tn = (uint32_t)column(t + 1) * (uint32_t)sizeof(X);
 #pragma unroll
     for (int e = 0; e < E; e++) acc[e] = -0.0;
