@@ -353,7 +353,8 @@ typedef struct wk_launch {
                               right-hand sides through a window of that
                               many values per column; the rest of k (fewer
                               than one tile), and engines it does not fit,
-                              run as 4; from five right-hand sides where
+                              run as 4; from three right-hand sides (not
+                              four on 8,192 groups or more) where
                               neighbouring rows share their columns (block
                               matrices, WPK1, at most 84 steps) FP64
                               engines, and FP32 ones with WK_ACC_F64, run

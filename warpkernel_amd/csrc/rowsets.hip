@@ -351,6 +351,7 @@ void launch_set(const SpmvArgs &a, const SetArgs &w, dim3 grid, int32_t nwork, i
 
 template <class P, int OUT, class I>
 SetFn pick_set_e(int e) {
+  if (e == 1) return &launch_set<P, OUT, 1, I>;
   if (e == 2) return &launch_set<P, OUT, 2, I>;
   return &launch_set<P, OUT, 4, I>;
 }
@@ -360,7 +361,7 @@ SetFn pick_set_i(int e, bool narrow) {
   return narrow ? pick_set_e<P, OUT, uint16_t>(e) : pick_set_e<P, OUT, int32_t>(e);
 }
 
-// e: right-hand sides per lane, a quarter of the k-tile (2 or 4).  Kr columns
+// e: right-hand sides per lane, a quarter of the k-tile (1, 2 or 4).  Kr columns
 // are always int32: a set's span reaches over the whole numbering.
 SetFn pick_set(int prec, int out, int e, bool narrow) {
   if (prec == 0) {
@@ -381,13 +382,13 @@ constexpr double kSetRows = 2.0;
 bool launch_rowsets(const DevLayout &D, int prec, int out, const SpmvArgs &a0, int32_t k, int32_t remap,
                     hipStream_t stream) {
   const bool kr = out == OUT_RUNX;
-  if (!D.rs_waves || D.win_max <= 0 || prec == 1 || k < kRowSetColumns || (kr && !D.rs_cols_kr)) return false;
+  if (!D.rs_waves || D.win_max <= 0 || prec == 1 || !row_sets_take(D, k) || (kr && !D.rs_cols_kr)) return false;
   SpmvArgs a = a0;
   if (!row_sets_reach(D, prec == 0 ? WK_F64 : WK_F32, a.ldx)) return false;
-  // Tiles of 8 or 16 columns.  The widest that k fills: it costs one pass
+  // Tiles of 4, 8 or 16 columns.  The widest that k fills: it costs one pass
   // over a wave's columns, and 16 FP64 values are a whole 128-byte line of x
   // (hex elasticity 64^3 k=32, 16-column tiles 382 us, 8-column ones 506).
-  const int e = k <= 8 ? 2 : 4;
+  const int e = k <= 4 ? 1 : k <= 8 ? 2 : 4;
   SetFn fn = pick_set(prec, out, e, D.rs_narrow);
   const SetArgs w{static_cast<const SetRec *>(D.rs_rec), kr ? D.rs_cols_kr : D.rs_cols, D.rs_waves};
   const int32_t ntiles = (k + 4 * e - 1) / (4 * e);

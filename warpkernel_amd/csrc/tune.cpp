@@ -35,17 +35,17 @@ const DevLayout &layout_for(const wk_engine *E, int32_t op) { return op == WK_OP
 
 // Whether stage 6 is the row sets.
 bool row_sets_run(const DevLayout &D, int32_t dtype, int32_t k, int32_t sums) {
-  return D.rs_waves > 0 && D.win_max > 0 && k >= kRowSetColumns && (dtype == WK_F64 || sums == WK_ACC_F64);
+  return D.rs_waves > 0 && D.win_max > 0 && row_sets_take(D, k) && (dtype == WK_F64 || sums == WK_ACC_F64);
 }
 
-// The sums of an FP32 engine that is not told: FP64 ones from kRowSetColumns where
+// The sums of an FP32 engine that is not told: FP64 ones from kRowSetDefault where
 // the layout has row sets, whichever kernel runs, so that they depend on k and the
 // matrix's structure and not on its size (they did: compensated up to k = 8 from
 // 8,192 groups, where 64^3 k=5 took 186 us against 122 here).  Exact products:
 // closer to the exact result than the compensated sums (1e-16 against 2e-14
 // normwise on 32^3), and faster (32^3 k=8 13.7 us against 23.5).
 int32_t default_sums(const DevLayout &D, int32_t k) {
-  return D.rs_waves > 0 && k >= kRowSetColumns ? WK_ACC_F64 : WK_ACC_TWOSUM;
+  return D.rs_waves > 0 && k >= kRowSetDefault ? WK_ACC_F64 : WK_ACC_TWOSUM;
 }
 
 // Where the row sets beat the layout's other kernels, by the rows a wave sums (8
@@ -57,6 +57,10 @@ int32_t default_sums(const DevLayout &D, int32_t k) {
 //   6.7; 468 groups, n 4 k=8 4.0 / 3.9), and the shortest above (n 2 k=12 23.3 / 30.1,
 //   n 4 42.2 / 29.9); FP32 values with FP64 sums longer ones on large layouts
 //   (3,750 groups, n 18 k=5 15.7 / 18.7; 936 groups, n 6 5.8 / 5.8);
+//   two, the largest layouts: whole window tiles, and k = 5 (n 18, 4,005 groups k=8 25.1 /
+//   23.0, 6,133 32.7 / 39.3, 8,002 41.2 / 51.0, k=12 68.7 / 73.2, but k=5 55.9 / 46.4, k=7
+//   94.3 / 50.5, k=16 107 / 82; 25,313 groups k=8 138 / 184, k=5 155 / 176; n 54, 8,192
+//   groups, k=8 106 / 100);
 //   three, large layouts: the shortest (3,750 groups, d 3: n 3 k=5 13.1 / 16.8, n 6 17.2 /
 //   16.8; FP32 n 3 10.5 / 14.6, n 6 14.3 / 14.6);
 //   up to three and fewer than 4 entries: k = 8, one tile of the direct kernel (249
@@ -67,6 +71,9 @@ bool row_sets_pay(const DevLayout &D, int32_t dtype, int32_t k, double mean_len)
   const bool f64 = dtype == WK_F64;
   const double rows = (double)D.nznrows / (double)D.rs_waves;
   const bool two = rows < 10.0, three = rows < 14.0;  // at most
+  if (two && mean_len < 32.0 && D.ngroups >= 5120 &&
+      ((k < 16 && k % 4 == 0) || (k == 5 && D.ngroups >= 10240)))
+    return false;
   if (k >= 9) return !(two && mean_len < 4.0 && D.ngroups >= 640);
   if (!f64 && D.ngroups >= 8192) return false;
   if (k == 8 && three && mean_len < 4.0) return false;
@@ -450,7 +457,7 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
     }
   }
   if (dtype != WK_F64) c.accumulate = sums != kDefaultSums ? sums : default_sums(D, k);
-  if (win_ok && row_sets_run(D, dtype, k, c.accumulate) && row_sets_pay(D, dtype, k, mean_len) &&
+  if (win_ok && k >= kRowSetDefault && row_sets_run(D, dtype, k, c.accumulate) && row_sets_pay(D, dtype, k, mean_len) &&
       row_sets_reach(D, dtype, ldx)) {
     // row sets on the matrix cores (stage 6, rowsets.hip), all of k in one
     // launch.  Hex elasticity, FP64: 32^3 k=5 18.1 us against 36.4, k=8 18.7
@@ -463,6 +470,8 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
     c.waves_per_block = 1;
     c.rows_per_lane = 1;
     c.xcd_remap = 1;
+  } else if (c.stage_lds == 6 && row_sets_run(D, dtype, k, c.accumulate)) {
+    c.stage_lds = 8;  // the register kernel, as chosen above
   }
   // as the launcher uses it (a masked last tile where the windows run it)
   c.k_tile = std::min(c.k_tile, masked ? pow2_at_least(std::max(1, k)) : pow2_at_most(std::max(1, k)));

@@ -249,9 +249,17 @@ void row_sets_finish(wk_engine *E, DevLayout &D, const uint64_t *starts, uint32_
 bool deltas_begin(wk_engine *E, DevLayout &D, std::vector<uint32_t> &off, uint32_t *fits, uint32_t *dev_off,
                   hipStream_t stream);
 void deltas_finish(wk_engine *E, DevLayout &D, const uint32_t *fits);
-// Right-hand sides from which the row sets run: below, the windows read less (hex
-// elasticity 64^3 k=4 118 us against 175; 32^3 17.5 either way).
-constexpr int32_t kRowSetColumns = 5;
+// Right-hand sides from which stage 6 is the row sets: with two, and with four
+// columns on large layouts, the windows read less (hex elasticity 64^3, 12,874
+// groups, stage 6 k=2 111 us by the windows and 174 by the row sets, k=4 154 and 177,
+// k=3 250 and 177; 32^3, 1,685 groups, k=2 16.1 and 17.9, k=4 23.0 and 18.2).
+constexpr int32_t kRowSetColumns = 3;
+inline bool row_sets_take(const DevLayout &D, int32_t k) {
+  return k >= kRowSetColumns && (k != 4 || D.ngroups < 8192);
+}
+// And from which they may be the default (64^3 k=4 118 us by the default's windows,
+// 32^3 17.5 either way).
+constexpr int32_t kRowSetDefault = 5;
 // Whether their 32-bit byte offsets reach every x (columns of an array of ldx).
 inline bool row_sets_reach(const DevLayout &D, int32_t dtype, int64_t ldx) {
   return ldx <= (int64_t)UINT32_MAX / (dtype == WK_F64 ? 8 : 4) / (D.ncols > 0 ? D.ncols : 1);
