@@ -73,6 +73,29 @@ def test_update_values_of_long_rows(name, variant, dtype, adjoint):
     eng.close()
 
 
+@pytest.mark.parametrize("name", ["short_4", "short_8", "column_and_row"])
+@pytest.mark.parametrize("variant", [1, 2])
+def test_update_values_of_narrow_groups(name, variant):
+    """Group width 32, short rows (one wave a group) and long ones, both layouts."""
+    say(f"[gpu] update narrow {name} {variant}")
+    m = CASES[name]
+    s = structure(32) if variant == 1 else structure2(32)
+    s.scan(m.nnz, m.nrows, m.vals, m.rowptr, m.colind, *([] if variant == 1 else [5]))
+    eng = engine(s, m.vals, m.colind, adjoint=True)
+    new = np.random.default_rng(9).uniform(-1, 1, m.nnz)
+    eng.update_values(dev(new))
+    pv, _ = s.process_host(new, m.colind)
+    assert np.array_equal(eng.download(capi.WK_ENGINE_VALUES), pv)
+    other = engine(s, new, m.colind, adjoint=True)
+    dy = dev(fe.uniform_x(m.nrows, seed=4))
+    a, b = (torch.full((m.ncols,), float("nan"), dtype=torch.float64, device="cuda") for _ in range(2))
+    eng.run_adjoint(dy, a)
+    other.run_adjoint(dy, b)
+    assert torch.equal(a, b)
+    other.close()
+    eng.close()
+
+
 def test_one_long_row_does_not_set_the_time():
     """200,000 rows of 9 entries, with and without one of 100,000 (5% more
     entries): within a factor of ten of each other, 50 us aside."""

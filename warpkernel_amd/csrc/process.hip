@@ -139,10 +139,11 @@ void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
   // group in two turns (hex elasticity, 81 entries: 48^3 residual with new values
   // 129.1 -> 122.1 us, 123.2 with 32 steps and eight waves; 16^3 update 5.9 -> 5.1;
   // but hex diffusion 60^3, 27 entries, 16.1 -> 17.4, and FP32 elasticity 28^3 8.4
-  // -> 9.0)
+  // -> 9.0).  Width 32 knows two tiles (tets 96^3 at threshold 5, both layouts, 174 us by
+  // the maps, 238 with 32 steps, 148 here)
   const int64_t slots = (int64_t)D.W * D.ngroups;
   const bool many = D.ngroups >= 4096;
-  const int steps = D.W != 64                                       ? 32
+  const int steps = D.W != 64 ? (many && D.allocate_nz <= 8 * slots ? 8 : 32)
                     : many && D.allocate_nz <= 4 * slots            ? 4
                     : many && D.allocate_nz <= 8 * slots            ? 8
                     : D.allocate_nz <= 16 * slots                   ? 16
@@ -175,7 +176,7 @@ void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
   const int64_t blocks = (int64_t)u.ngroups + u.nblocks_t;
   if (blocks > INT32_MAX) fail(WK_ERR_LIMIT, "grid too large");
   if (blocks == 0) return;
-  const auto kernel = D.W != 64     ? update_kernel<T, 32, 32, kThreads>
+  const auto kernel = D.W != 64     ? (steps == 8 ? update_kernel<T, 32, 8, 64> : update_kernel<T, 32, 32, kThreads>)
                       : steps == 4  ? update_kernel<T, 64, 4, 64>
                       : steps == 8  ? update_kernel<T, 64, 8, 64>
                       : steps == 16 ? update_kernel<T, 64, 16, kThreads>
