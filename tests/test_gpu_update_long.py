@@ -24,13 +24,13 @@ def dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
-def matrix(nrows, lens, column=0, seed=3):
-    """lens[r % len(lens)] entries in row r near the diagonal; column > 0: an entry
+def matrix(nrows, lens, column=0, seed=3, width=30):
+    """lens[r % len(lens)] entries in row r within `width` of the diagonal; column > 0: an entry
     of column 0 in each of the first `column` rows too."""
     rng = np.random.default_rng(seed)
     n = np.asarray(lens, np.int64)[np.arange(nrows) % len(lens)]
     rows = np.concatenate([np.repeat(np.arange(nrows), n), np.arange(column)])
-    near = np.clip(rows + rng.integers(-30, 31, rows.size), 1, nrows - 1)
+    near = np.clip(rows + rng.integers(-width, width + 1, rows.size), 1, nrows - 1)
     cols = np.where(np.arange(rows.size) < n.sum(), near, 0)
     order = np.lexsort((cols, rows))
     rp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=nrows))]).astype(np.int32)
@@ -43,6 +43,7 @@ CASES = {
     "dense": matrix(150, [900]),
     "column": matrix(6000, [5, 7], 6000),
     "column_and_row": matrix(6000, [4000] + [5] * 5999, 3000),
+    "scattered": matrix(70000, [15, 17], width=300),  # 1.1M entries, far apart in the transposed layout
     "short_4": matrix(64 * 4096 + 7, [1, 4, 3]),
     "short_8": matrix(64 * 4096 + 7, [5, 8, 1, 7]),
 }

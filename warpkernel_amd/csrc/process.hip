@@ -3,16 +3,16 @@
 // alone, on the device.
 //
 // Layouts whose lanes hold runs of CSR entries (every forward layout without
-// the row sort) and whose longest group is no bottleneck: one block per group
-// reads its rows' entries 4 to 64 at a time, turns them around in LDS and writes
-// whole steps.  It streams 16 bytes per FP64 entry, both ways in whole lines,
+// the row sort), unless small or with a group that is a bottleneck: one block per
+// group reads its rows' entries 4 to 64 at a time, turns them around in LDS and
+// writes whole steps.  It streams 16 bytes per FP64 entry, both ways in whole lines,
 // with no index array.  (One thread per entry writing through the CSR-to-slot map
 // put 8 bytes into each 128-byte line: hex elasticity 48^3, 27.4M entries, 305 us
-// against 77.)  The transposed layout, unless padded much, reads the entry of each
-// slot instead: indices and values written in order, the 8-byte reads land on
-// lines that the same group's other steps read too (hex diffusion 48^3, both
-// layouts 31 us as two scatters, 23 here in one launch).  The others go through
-// the map.
+// against 77.)  The transposed layout, where its entries lie near each other and
+// few slots are pads, reads the entry of each slot instead: indices and values
+// written in order, the 8-byte reads land on lines that the same group's other
+// steps read too (hex diffusion 48^3, both layouts 31 us as two scatters, 23 here
+// in one launch).  The others go through the map.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -104,8 +104,7 @@ __global__ __launch_bounds__(TH) void update_kernel(UpdateArgs u) {
     gather_slots<T, TH>(u, work_id(b - u.ngroups, u.nblocks_t, 1));
 }
 
-// Layouts whose lanes hold no runs (the row sort), with a group much longer than
-// its share of the entries, or padded much: entry i to slot[i].
+// The other layouts: entry i to slot[i].
 template <class T>
 __global__ __launch_bounds__(kThreads) void scatter_kernel(const T *__restrict__ src,
                                                            const uint32_t *__restrict__ slot,
@@ -140,23 +139,34 @@ void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
   // 129.1 -> 122.1 us, 123.2 with 32 steps and eight waves; 16^3 update 5.9 -> 5.1;
   // but hex diffusion 60^3, 27 entries, 16.1 -> 17.4, and FP32 elasticity 28^3 8.4
   // -> 9.0).  Width 32 knows two tiles (tets 96^3 at threshold 5, both layouts, 174 us by
-  // the maps, 238 with 32 steps, 148 here)
+  // the maps, 238 with 32 steps, 148 with 8)
   const int64_t slots = (int64_t)D.W * D.ngroups;
   const bool many = D.ngroups >= 4096;
-  const int steps = D.W != 64 ? (many && D.allocate_nz <= 8 * slots ? 8 : 32)
+  const int steps = D.W != 64 ? (D.allocate_nz <= 16 * slots ? 8 : 32)
                     : many && D.allocate_nz <= 4 * slots            ? 4
                     : many && D.allocate_nz <= 8 * slots            ? 8
                     : D.allocate_nz <= 16 * slots                   ? 16
                     : sizeof(T) == 4 || D.allocate_nz <= 32 * slots ? 32
                                                                     : 64;
   const int threads = steps <= 8 ? 64 : steps == 64 ? 512 : kThreads;
-  // A block turns its group's steps one tile after another, 0.7 to 1.5 us each,
-  // while the map takes 11 us per million FP64 entries, 6 per million FP32 ones,
-  // whatever the rows: layouts with a group too long for its share keep the map
+  // A block turns its group's steps one tile after another, about 1.1 us each, while
+  // the map takes 11 us per million FP64 entries of long rows, 6 per million FP32
+  // ones: layouts with a group too long for its share of the entries keep the map
   // (200,000 rows of 9 entries and one of 100,000: 9.8 us, 1,568 turned; 64 of 8,000
-  // 13.6, 419; 1,500 rows of 1,500, 24 groups, 25.4, 39.2; but 20,000 of 500 147, 37.9)
+  // 13.6, 419; 1,500 rows of 1,500, 24 groups, 25.4, 39.2; but 20,000 of 500 147, 37.9;
+  // 4,096 of 300, FP64 16.4, 10.3, FP32 11.4, 13.2; in a graph, 1,000 rows of 81 2.9, 4.6).
+  // So do small ones, whose map stays in L2, unless the transposed layout takes its
+  // values in the same launch (in a graph: 20,000 rows of 9 entries 2.8, 3.0, of 16
+  // 3.0, 3.2; elasticity 8^3 3.3, 4.6; both layouts of the 9 6.1 as two maps, 4.5), and
+  // larger ones of the shortest rows, whose groups hold too little (400,000 rows of 2
+  // 3.9, 4.8, FP32 3.1, 4.3; of 4 7.4, 6.1, FP32 4.2, 4.8; 100,000 of 9 5.1, 4.6)
+  constexpr bool f64 = sizeof(T) == 8;
   const int64_t turns = ((int64_t)D.longest + steps - 1) / steps;
-  if (D.lane_src && turns <= 3 + E->nnz / (sizeof(T) == 8 ? 131072 : 262144)) {
+  const bool shared = E->has_adj && E->adj.src_of_slot;
+  const bool by_map = !D.lane_src || turns > 1 + E->nnz / (f64 ? 131072 : 262144) ||
+                      (!shared && (E->nnz <= 327680 ||
+                                   (D.allocate_nz <= 6 * slots && E->nnz <= (f64 ? 1 << 20 : 1 << 21))));
+  if (!by_map) {
     u.dst = D.vals;
     u.lane_src = reinterpret_cast<const int2 *>(D.lane_src);
     u.warp_offsets = D.warp_offsets;
@@ -165,7 +175,7 @@ void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
   } else {
     scatter<T>(D, vals, E->nnz, s);
   }
-  if (E->has_adj && E->adj.src_of_slot) {
+  if (shared) {
     u.dst_t = E->adj.vals;
     u.src_of_slot = E->adj.src_of_slot;
     u.slots_t = E->adj.allocate_nz;

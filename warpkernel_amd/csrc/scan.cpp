@@ -276,6 +276,33 @@ bool lane_sources(const wk_layout &L, std::vector<int32_t> &src) {
   return runs && entries == L.nz;
 }
 
+// Up to 2 slots per entry (a dense column of A pads its group: one of 100,000 entries
+// over 1.9M, 4.3 slots per entry, both layouts 25.7 us by maps, 68.6 slot by slot), and
+// small, or with at most 0.6 64-byte lines of FP64 values per entry over 1,024 slots (64
+// runs of them): finite-element meshes have 0.28 to 0.46 and gain (transposed part, hex
+// elasticity 40^3 96 us by the map and 79 slot by slot, tets 80^3 43 and 41, FP32 23 and
+// 17), bands of random columns, whose rows of A^T are sorted by length over the whole
+// matrix, 0.68 to 0.88 and lose (100,000 rows of 40 38 and 61, FP32 27 and 44;
+// but 20,000 of 40 9.6 and 9.1), random numberings 0.97 to 0.99 (tets 80^3 149 and 144,
+// FP32 98 and 121, but 40^3 12.3 and 11.5, FP32 9.9 and 6.9).
+bool gather_pays(const wk_layout &L, const std::vector<int32_t> &src) {
+  if (L.allocate_nz > 2 * L.nz) return false;
+  if (L.nz <= 1 << 20) return true;
+  constexpr int64_t kRuns = 64, kRun = 1024;
+  int64_t lines = 0, entries = 0;
+  std::vector<int32_t> e;
+  for (int64_t r = 0; r < kRuns; r++) {
+    const int64_t s0 = (L.allocate_nz - kRun) / (kRuns - 1) * r;
+    e.clear();
+    for (int64_t s = s0; s < s0 + kRun; s++)
+      if (src[(size_t)s] >= 0) e.push_back(src[(size_t)s] / 8);
+    entries += (int64_t)e.size();
+    std::sort(e.begin(), e.end());
+    lines += std::unique(e.begin(), e.end()) - e.begin();
+  }
+  return (double)lines <= 0.6 * (double)entries;
+}
+
 template <class T>
 void process_host(const wk_layout &L, const double *vals, const int32_t *colind, T *pvals,
                   int32_t *pcols) {

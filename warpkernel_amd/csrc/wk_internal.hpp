@@ -96,7 +96,7 @@ struct DevLayout {
                                      // transposed ones without src_of_slot)
   // GPU process: the first CSR entry and the entries of each lane of each group
   // (forward layouts without the row sort), or every slot's CSR entry, -1 for a
-  // pad (transposed layouts of at most kGatherPads slots per entry)
+  // pad (transposed layouts where gather_pays)
   int32_t *lane_src = nullptr;       // [ngroups * W * 2]
   int32_t *src_of_slot = nullptr;    // [allocate_nz]
   std::vector<uint32_t> h_max_nz_rows;  // host copy (batch work partition)
@@ -215,11 +215,9 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
                  const void *x, int64_t ldx, double *y, int64_t ldy, const double *b,
                  int64_t ldb, int32_t k, hipStream_t stream);
 
-// Slots per entry up to which a transposed layout's slots take their values one by
-// one: a long row among short ones (a dense column of A) pads its group, and its
-// entries find their slots through the map instead (one column of 100,000 entries
-// over 1.9M, 4.3 slots per entry, both layouts 25.7 us by maps, 68.6 slot by slot).
-constexpr int64_t kGatherPads = 2;
+// Whether a transposed layout's slots take their values one by one (src: every slot's
+// CSR entry, -1 for a pad), or the entries find their slots through the map.
+bool gather_pays(const wk_layout &L, const std::vector<int32_t> &src);
 // New CSR values (of the engine's type) into its forward and, where it has one,
 // transposed layout (GPU process).
 void launch_update_values(const wk_engine *E, const void *vals_csr, hipStream_t stream);
