@@ -227,7 +227,7 @@ void upload_layout(wk_engine *E, DevLayout &D, const wk_layout &L, const double 
     src.assign((size_t)L.allocate_nz, -1);
     for (int64_t i = 0; i < L.nz; i++) src[slot_of_nz[i]] = (int32_t)i;
   }
-  if (&D == &E->adj && gather_pays(L, src)) {
+  if (&D == &E->adj && gather_pays(L, dtype, src)) {
     D.src_of_slot = dev_upload(E, src.data(), (int64_t)src.size(), s);
   } else {
     D.slot_of_nz = dev_upload(E, slot_of_nz ? slot_of_nz : L.reorder_rows.data(), L.nz, s);

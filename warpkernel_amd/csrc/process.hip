@@ -142,7 +142,7 @@ void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
   // the maps, 238 with 32 steps, 148 with 8)
   const int64_t slots = (int64_t)D.W * D.ngroups;
   const bool many = D.ngroups >= 4096;
-  const int steps = D.W != 64 ? (D.allocate_nz <= 16 * slots ? 8 : 32)
+  const int steps = D.W != 64 ? (D.ngroups >= 2048 && D.allocate_nz <= 16 * slots ? 8 : 32)
                     : many && D.allocate_nz <= 4 * slots            ? 4
                     : many && D.allocate_nz <= 8 * slots            ? 8
                     : D.allocate_nz <= 16 * slots                   ? 16
@@ -154,7 +154,8 @@ void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
   // ones: layouts with a group too long for its share of the entries keep the map
   // (200,000 rows of 9 entries and one of 100,000: 9.8 us, 1,568 turned; 64 of 8,000
   // 13.6, 419; 1,500 rows of 1,500, 24 groups, 25.4, 39.2; but 20,000 of 500 147, 37.9;
-  // 4,096 of 300, FP64 16.4, 10.3, FP32 11.4, 13.2; in a graph, 1,000 rows of 81 2.9, 4.6).
+  // 4,096 of 300, FP64 16.4, 10.3, FP32 11.4, 13.2; in a graph, 1,000 rows of 81 2.9, 4.6,
+  // but FP32 elasticity 12^3, both layouts in one launch, 9.3, 5.8).
   // So do small ones, whose map stays in L2, unless the transposed layout takes its
   // values in the same launch (in a graph: 20,000 rows of 9 entries 2.8, 3.0, of 16
   // 3.0, 3.2; elasticity 8^3 3.3, 4.6; both layouts of the 9 6.1 as two maps, 4.5), and
@@ -163,7 +164,7 @@ void update_values(const wk_engine *E, const void *vals, hipStream_t s) {
   constexpr bool f64 = sizeof(T) == 8;
   const int64_t turns = ((int64_t)D.longest + steps - 1) / steps;
   const bool shared = E->has_adj && E->adj.src_of_slot;
-  const bool by_map = !D.lane_src || turns > 1 + E->nnz / (f64 ? 131072 : 262144) ||
+  const bool by_map = !D.lane_src || turns > (shared ? 3 : 1) + E->nnz / (f64 ? 131072 : 262144) ||
                       (!shared && (E->nnz <= 327680 ||
                                    (D.allocate_nz <= 6 * slots && E->nnz <= (f64 ? 1 << 20 : 1 << 21))));
   if (!by_map) {

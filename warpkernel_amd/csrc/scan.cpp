@@ -276,16 +276,19 @@ bool lane_sources(const wk_layout &L, std::vector<int32_t> &src) {
   return runs && entries == L.nz;
 }
 
-// Up to 2 slots per entry (a dense column of A pads its group: one of 100,000 entries
-// over 1.9M, 4.3 slots per entry, both layouts 25.7 us by maps, 68.6 slot by slot), and
-// small, or with at most 0.6 64-byte lines of FP64 values per entry over 1,024 slots (64
-// runs of them): finite-element meshes have 0.28 to 0.46 and gain (transposed part, hex
-// elasticity 40^3 96 us by the map and 79 slot by slot, tets 80^3 43 and 41, FP32 23 and
-// 17), bands of random columns, whose rows of A^T are sorted by length over the whole
-// matrix, 0.68 to 0.88 and lose (100,000 rows of 40 38 and 61, FP32 27 and 44;
-// but 20,000 of 40 9.6 and 9.1), random numberings 0.97 to 0.99 (tets 80^3 149 and 144,
-// FP32 98 and 121, but 40^3 12.3 and 11.5, FP32 9.9 and 6.9).
-bool gather_pays(const wk_layout &L, const std::vector<int32_t> &src) {
+// Small layouts, where both layouts' values then go in one launch (in a graph, 1,000 rows
+// of 9 entries 4.2 us by two maps, 2.9).  Larger ones of up to 2 slots per entry (a dense
+// column of A pads its group: one of 100,000 entries over 1.9M, 4.3 slots per entry, both
+// layouts 25.7 us by maps, 68.6 slot by slot) with at most 0.6 64-byte lines of FP64
+// values per entry over 1,024 slots (64 runs of them; 0.7 for FP32): finite-element
+// meshes have 0.28 to 0.46 and gain (transposed part, hex elasticity 40^3 96 us by the
+// map and 79 slot by slot, tets 80^3 43 and 41, FP32 23 and 17), bands of random columns,
+// whose rows of A^T are sorted by length over the whole matrix, 0.68 to 0.88 and lose
+// (100,000 rows of 40 38 and 61, FP32 27 and 44; 400,000 of 4, 0.68, 14.9 and 16.5, FP32
+// 12.2 and 10.4; but 20,000 of 40 9.6 and 9.1), random numberings 0.97 to 0.99 (tets 80^3
+// 149 and 144, FP32 98 and 121, but 40^3 12.3 and 11.5, FP32 9.9 and 6.9).
+bool gather_pays(const wk_layout &L, int32_t dtype, const std::vector<int32_t> &src) {
+  if (L.allocate_nz <= 1 << 20) return true;
   if (L.allocate_nz > 2 * L.nz) return false;
   if (L.nz <= 1 << 20) return true;
   constexpr int64_t kRuns = 64, kRun = 1024;
@@ -300,7 +303,7 @@ bool gather_pays(const wk_layout &L, const std::vector<int32_t> &src) {
     std::sort(e.begin(), e.end());
     lines += std::unique(e.begin(), e.end()) - e.begin();
   }
-  return (double)lines <= 0.6 * (double)entries;
+  return (double)lines <= (dtype == WK_F64 ? 0.6 : 0.7) * (double)entries;
 }
 
 template <class T>

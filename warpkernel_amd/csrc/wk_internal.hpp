@@ -217,7 +217,7 @@ void launch_spmv(const DevLayout &D, int32_t dtype, const wk_launch &cfg, int ou
 
 // Whether a transposed layout's slots take their values one by one (src: every slot's
 // CSR entry, -1 for a pad), or the entries find their slots through the map.
-bool gather_pays(const wk_layout &L, const std::vector<int32_t> &src);
+bool gather_pays(const wk_layout &L, int32_t dtype, const std::vector<int32_t> &src);
 // New CSR values (of the engine's type) into its forward and, where it has one,
 // transposed layout (GPU process).
 void launch_update_values(const wk_engine *E, const void *vals_csr, hipStream_t stream);
