@@ -13,10 +13,12 @@
 // a k-tile's window leaves a few waves per CU (hex elasticity 32^3 k=16: LDS
 // 23% busy at 1.65 waves per SIMD).  Here one read of x serves the set's rows,
 // the values stay in registers whatever k, and no window limits residency
-// (12 or 16 waves per CU).  Hex elasticity FP64, against the window kernels:
-// 32^3 k=16 58.4 -> 25.1 us, k=32 100 -> 38.4; 64^3 k=16 421 -> 248, k=32
-// 803 -> 382.  What bounds it: a wave first waits for its record, then for its
-// values (64^3 k=4: 61 us without the values, 133 without x, 175 with both);
+// (12 or 16 waves per CU).  Hex elasticity FP64, against the window kernels, one
+// set of inputs repeated: 32^3 k=16 58.4 -> 25.1 us, k=32 100 -> 38.4; 64^3 k=16
+// 421 -> 248, k=32 803 -> 382 (other inputs from pass to pass: 32^3 k=16 58.5 ->
+// 33.6, 48^3 k=32 365 -> 167).  What bounds it: a wave first waits for its
+// record, then for its values (64^3 k=4: 61 us without the values, 133 without
+// x, 175 with both);
 // from k = 16 on the reads of x through L1, 67 us per 8 columns at 64^3 where
 // the matrix instructions alone take 18.  Measured and not kept: x through an
 // LDS window filled by direct-to-LDS loads (64^3 k=8 221 us, k=32 489), values

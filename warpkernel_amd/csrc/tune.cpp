@@ -460,8 +460,9 @@ wk_launch heuristic_launch(const DevLayout &D, int32_t dtype, int32_t k, bool kr
   if (win_ok && k >= kRowSetDefault && row_sets_run(D, dtype, k, c.accumulate) && row_sets_pay(D, dtype, k, mean_len) &&
       row_sets_reach(D, dtype, ldx)) {
     // row sets on the matrix cores (stage 6, rowsets.hip), all of k in one
-    // launch.  Hex elasticity, FP64: 32^3 k=5 18.1 us against 36.4, k=8 18.7
-    // against 30.9, k=16 25.1 against 58.4, k=32 38.4 against 100; 64^3 k=5
+    // launch.  Hex elasticity, FP64, one set of inputs repeated: 32^3 k=5 18.1 us
+    // against 36.4, k=8 18.7 against 30.9, k=16 25.1 against 58.4 (other inputs
+    // from pass to pass 33.6 against 58.5), k=32 38.4 against 100; 64^3 k=5
     // 176 against 194, k=8 181 against 204, k=16 248 against 421, k=32 382
     // against 803.  FP32 values with FP64 sums: 32^3 k=8 13.7 us, 48^3 36.4.
     c.stage_lds = 6;

@@ -145,7 +145,9 @@ struct DevLayout {
   // rows or more on average
   void *rs_rec = nullptr;        // [rs_waves] four sets each: slots, rows, least columns
   void *rs_cols = nullptr;       // their columns in the kernel's lane order: uint16 from
-                                 // each set's least column, or int32
+                                 // each set's least column, or int32 for the whole
+                                 // layout where one set (pads are column 0) spans
+                                 // more than 65,535
   void *rs_cols_kr = nullptr;    // the same in Kr numbering (int32)
   bool rs_narrow = false;        // rs_cols holds uint16
   int32_t rs_waves = 0;          // 0: no row sets
